@@ -313,16 +313,24 @@ typedef struct {
 int g3k_rows(const g3k_rows_args *a, void *stream);
 
 /* Batched projection on MFMA: C[n][m] = sum_k X[n][k] W[m][k] for N tokens,
- * X given as bf16 planes x_hi + x_lo [N][ldx], W bf16 [M][K] (K % (32 ksplit)
- * == 0, M % 4 == 0).  mode 0: n_mat (1..3) matrices sharing X, each written
- * to C[j] [N][ldc[j]] fp32; with ksplit S > 1, split s covers k in
- * [s K / S, (s + 1) K / S) and writes its partial product to C[j] +
- * s * split_stride (floats), for the consumer to add.  mode G3K_MV_GEGLU
- * (ksplit 1): W[0] = gate, W[1] = up (same M); gelu_tanh(gate) * up is
- * written as bf16 planes h_hi + h_lo [N][ldh]. */
+ * X given as bf16 planes x_hi + x_lo [N][ldx], W bf16 [M][K] (K % 32 == 0,
+ * M % 4 == 0).  mode 0: n_mat (1..3) matrices sharing X, each written to C[j]
+ * [N][ldc[j]] fp32.  mode G3K_MV_GEGLU: W[0] = gate, W[1] = up (same M);
+ * gelu_tanh(gate) * up is written as bf16 planes h_hi + h_lo [N][ldh].
+ * kind: G3K_GEMM_TILE, 256 weight rows x 128 tokens per workgroup; _WIDE and
+ * _NARROW, few tokens, 256 and 64 rows; _GATE, GEGLU over many tokens.
+ * ksplit S > 1 (plain, or GEGLU of _WIDE / _NARROW): split s sums its share of
+ * the 64-wide chunks of k.  With part [S][N][sum of M] the partial products
+ * go there and a second launch adds them in split order (GEGLU of _WIDE /
+ * _NARROW: required); without it they go to C[j] + s * split_stride
+ * (floats), for the consumer to add.  g3k_gemm_plan picks kind and ksplit
+ * (consumer_adds: the partial products go to C). */
+enum { G3K_GEMM_TILE = 0, G3K_GEMM_WIDE = 1, G3K_GEMM_NARROW = 2, G3K_GEMM_GATE = 3 };
+void g3k_gemm_plan(int N, int K, int n_mat, const int *M, int geglu, int consumer_adds, int n_cu, int *kind,
+                   int *ksplit);
 typedef struct {
     const uint16_t *x_hi, *x_lo;
-    int N, K, ldx, n_mat, mode, ksplit;
+    int N, K, ldx, n_mat, mode, kind, ksplit;
     long long split_stride;
     const uint16_t *W[G3K_MATVEC_MAX];
     int M[G3K_MATVEC_MAX];
@@ -330,6 +338,7 @@ typedef struct {
     int ldc[G3K_MATVEC_MAX];
     uint16_t *h_hi, *h_lo;
     int ldh;
+    float *part;
 } g3k_gemm_args;
 
 int g3k_gemm(const g3k_gemm_args *a, void *stream);

@@ -14,6 +14,23 @@
 #define G3K_WAIT_VMEM() asm volatile("s_waitcnt vmcnt(0)" ::: "memory")
 #endif
 
+// A workgroup barrier that leaves this wave's youngest n vector-memory
+// operations in flight (__syncthreads waits for all of them): everything
+// older has completed, LDS reads included, on every wave past it.
+#ifndef G3K_WAIT_BARRIER
+#define G3K_WAIT_BARRIER(n) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(n) : "memory")
+#endif
+
+// Keeps the memory operations before it before those after it, in the
+// compiler and its scheduler (no instruction).
+#ifndef G3K_ORDER_FENCE
+#define G3K_ORDER_FENCE()                 \
+    do {                                  \
+        asm volatile("" ::: "memory");    \
+        __builtin_amdgcn_sched_barrier(0); \
+    } while (0)
+#endif
+
 // The XCD this wave runs on: the hardware register XCC_ID (gfx940 and
 // later), whose low 4 bits number the XCDs.  The host-emulation build
 // defines it as the workgroup id mod 8.

@@ -12,24 +12,22 @@
 // with fp32 accumulation: twice the algorithmic MFMA work, within a few
 // 2^-17 of the reference's fp32 sgemm.
 //
-// Tiling.  Workgroup = 4 waves = a 128 (weight rows) x 128 (tokens) tile of
-// C; wave (wm, wn) owns 64 x 64 of it, 4 x 4 MFMA tiles of 16 x 16 (64
-// accumulator registers).  K advances 32 at a time: per stage the W tile and
-// the x_hi / x_lo tiles (128 rows x 32 k each, 8 KiB) move from global memory
-// straight into LDS with buffer -> LDS loads (buffer_load_dwordx4 ... lds, one
-// wave instruction = 1 KiB = 16 rows).  Rows beyond M or N read zero (the
-// buffer descriptor's range check), so ragged tiles need no masking until the
-// stores.  LDS rows are 64 B; within each 16-row group the four 16-byte
-// chunks of row r sit at slot 4 r + (c ^ (r / 4 % 4)), so a fragment read (16
-// rows, one chunk) touches all 64 banks once.  MFMA operands: A = W rows (lane
-// l: row l % 16, k 8 (l / 16) .. + 7), B = X rows in the same pattern; the
-// accumulator of lane l holds C rows m = 4 (l / 16) + i for token l % 16.
+// Tiling.  Three forms of gemm_kernel, picked by g3k_gemm_plan: Pairs (many
+// tokens), Stream in two widths (few tokens) and Gate (GEGLU over the most
+// tokens); each says what bounds it.  In all of them W and x tiles move
+// from global memory straight into LDS with buffer -> LDS loads
+// (buffer_load_dwordx4 ... lds, one wave instruction = 1 KiB).  Rows beyond M
+// or N read zero (the buffer descriptor's range check), so ragged tiles need
+// no masking until the stores.  A row's 16-byte pieces are XOR-swizzled by
+// row bits, so a fragment read (16 rows, one piece) spreads over the banks.
+// MFMA operands: A = W rows (lane l: row l % 16, k 8 (l / 16) .. + 7), B = X
+// rows in the same pattern; the accumulator of lane l holds C rows m = 4 (l /
+// 16) + i for token l % 16.
 //
 // Modes.  PLAIN: up to three weight matrices that share X in one launch (the
 // Q, K and V projections), each written as fp32 C [N][ldc].  GEGLU: the gate
-// and up matrices together; the epilogue computes gelu_tanh(gate) * up
-// (gemma3_transformer.c:741-745) and writes it as the bf16 hi / lo planes
-// that the down projection reads.
+// and up matrices together; gelu_tanh(gate) * up (gemma3_transformer.c:741-745)
+// is written as the bf16 hi / lo planes that the down projection reads.
 #include <hip/hip_runtime.h>
 
 #include "g3k.h"
@@ -87,41 +85,67 @@ __device__ __forceinline__ uint32_t bf16_rne(float f) {
     return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
 }
 
-// MT: 16-row MFMA tiles per wave along the weight rows (4 or 8).  The
-// workgroup's 4 waves sit 2 (rows) x 2 (tokens); the W region of a stage
-// holds 32 MT rows (GEGLU, MT = 8: 128 gate rows, then the same 128 up rows).
-// Wave (wm, wn) owns rows wm * 16 MT .. of the region (GEGLU: 64 gate rows and
-// the same 64 up rows) and tokens wn * 64 .. + 63.  Per 32-wide k step a wave
-// reads MT W fragments and 8 x fragments (4 hi, 4 lo) for 8 MT MFMAs.
-// blockIdx.z = k split: split s sums k in [s K / S, (s + 1) K / S) and writes
-// C + s * split_stride (the consumer adds the S partial products).
-template <bool GEGLU, int MT>
-__global__ __launch_bounds__(NT, 2) void gemm_kernel(g3k_gemm_args a) {
-    static_assert(!GEGLU || MT == 8, "GEGLU tiles pair 4 gate and 4 up tiles per wave");
-    constexpr int RW = 32 * MT;                          // W rows per stage
-    constexpr int W_B = RW * BK * 2;
+// Four values of token n at columns m.. as the bf16 hi / lo planes.
+__device__ __forceinline__ void store_planes(const g3k_gemm_args &a, int n, int m, float h0, float h1, float h2,
+                                             float h3) {
+    const float h[4] = {h0, h1, h2, h3};
+    uint32_t hi[4], lo[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        hi[i] = bf16_rne(h[i]);
+        lo[i] = bf16_rne(h[i] - __uint_as_float(hi[i] << 16));
+    }
+    const size_t o = (size_t)n * a.ldh + m;
+    *reinterpret_cast<uint2 *>(a.h_hi + o) = make_uint2(hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16));
+    *reinterpret_cast<uint2 *>(a.h_lo + o) = make_uint2(lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16));
+}
+
+// One buffer -> LDS fetch of 1 KiB, 16 bytes per lane.  soff (uniform) stays
+// below the buffer's size, so the range check covers voff + soff: a lane past
+// the end reads zero.
+__device__ __forceinline__ void fetch8(__amdgpu_buffer_rsrc_t rs, char *dst, uint32_t voff, uint32_t soff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr)dst, 16, voff, soff, 0, 0);
+}
+
+// Where matrix m's products of split z go, and their row stride: C, or with
+// a.part the columns of the matrices side by side, [split][N][sum of M].
+__device__ __forceinline__ float *out_base(const g3k_gemm_args &a, int m, int z, long long &ld) {
+    if (!a.part) {
+        ld = a.ldc[m];
+        return a.C[m] + (size_t)z * a.split_stride;
+    }
+    int col = 0;
+    ld = 0;
+    for (int j = 0; j < a.n_mat; j++) {
+        if (j < m) col += a.M[j];
+        ld += a.M[j];
+    }
+    return a.part + (size_t)z * a.N * ld + col;
+}
+
+// GEGLU over many tokens: 128 gate rows and the same 128 up rows x 128 tokens
+// per workgroup of 4 waves, two workgroups per CU (64 KiB of LDS each, two
+// stages of 32 k values).  Wave (wm, wn) owns 64 gate rows, the same 64 up
+// rows and tokens wn * 64 .. + 63; per k step it reads 8 W fragments and 8 x
+// fragments (4 hi, 4 lo) for 64 MFMAs.
+struct Gate {
+    static constexpr int THREADS = NT, WAVES = 2;
+    static __device__ void run(const g3k_gemm_args &a);
+};
+__device__ __forceinline__ void Gate::run(const g3k_gemm_args &a) {
+    constexpr int MT = 8;
+    constexpr int W_B = 2 * TILE_B;
     constexpr int STAGE_B = W_B + 2 * TILE_B;
     __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE_B];
 
-    // this workgroup's weight matrix and row block
-    constexpr int BMW = GEGLU ? RW / 2 : RW;             // matrix rows per workgroup
-    int bx = blockIdx.x, m_idx = 0;
-    if (!GEGLU) {
-        while (m_idx + 1 < a.n_mat && bx >= (a.M[m_idx] + BMW - 1) / BMW) {
-            bx -= (a.M[m_idx] + BMW - 1) / BMW;
-            m_idx++;
-        }
-    }
-    const int M = a.M[m_idx], K = a.K, N = a.N;
-    const int m0 = bx * BMW, n0 = blockIdx.y * BN;
-    const int kc = K / a.ksplit, kbeg = blockIdx.z * kc;
+    const int M = a.M[0], K = a.K, N = a.N;
+    const int m0 = blockIdx.x * 128, n0 = blockIdx.y * BN;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave & 1, wn = wave >> 1;
 
     const uint32_t wbytes = (uint32_t)((size_t)M * K * 2);
-    const __amdgpu_buffer_rsrc_t rw0 = rsrc(a.W[GEGLU ? 0 : m_idx], wbytes);
-    const __amdgpu_buffer_rsrc_t rw1 = rsrc(a.W[GEGLU ? 1 : m_idx], wbytes);
+    const __amdgpu_buffer_rsrc_t rw0 = rsrc(a.W[0], wbytes), rw1 = rsrc(a.W[1], wbytes);
     const uint32_t xbytes = (uint32_t)((size_t)N * a.ldx * 2);
     const __amdgpu_buffer_rsrc_t rxh = rsrc(a.x_hi, xbytes), rxl = rsrc(a.x_lo, xbytes);
 
@@ -133,28 +157,18 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(g3k_gemm_args a) {
 
     auto fetch = [&](int s, int k0) {
         char *st = smem + s * STAGE_B;
-        if (GEGLU) {
-            fetch_tile(rw0, st, m0, K, k0, wave, lane);
-            fetch_tile(rw1, st + TILE_B, m0, K, k0, wave, lane);
-        } else {
-#pragma unroll
-            for (int h = 0; h < RW / 128; h++) fetch_tile(rw0, st + h * TILE_B, m0 + 128 * h, K, k0, wave, lane);
-        }
+        fetch_tile(rw0, st, m0, K, k0, wave, lane);
+        fetch_tile(rw1, st + TILE_B, m0, K, k0, wave, lane);
         fetch_tile(rxh, st + W_B, n0, a.ldx, k0, wave, lane);
         fetch_tile(rxl, st + W_B + TILE_B, n0, a.ldx, k0, wave, lane);
     };
-    // W region row of the wave's tile mt
-    auto wrow = [&](int mt) {
-        if (GEGLU) return (mt >> 2) * 128 + wm * 64 + (mt & 3) * 16;
-        return wm * 16 * MT + mt * 16;
-    };
 
-    const int nk = kc / BK;
+    const int nk = K / BK;
     const int fr = lane & 15, fc = lane >> 4;
-    fetch(0, kbeg);
+    fetch(0, 0);
     for (int kt = 0; kt < nk; kt++) {
         __syncthreads();   // stage kt has landed; stage kt + 1's slot is free
-        if (kt + 1 < nk) fetch((kt + 1) & 1, kbeg + (kt + 1) * BK);
+        if (kt + 1 < nk) fetch((kt + 1) & 1, (kt + 1) * BK);
         const char *st = smem + (kt & 1) * STAGE_B;
         bf16x8 bh[4], bl[4];
 #pragma unroll
@@ -164,7 +178,8 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(g3k_gemm_args a) {
         }
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
-            const bf16x8 w = frag(st, wrow(mt) + fr, fc);
+            // W region row of the wave's tile mt: gate tiles 0..3, up tiles 4..7
+            const bf16x8 w = frag(st, (mt >> 2) * 128 + wm * 64 + (mt & 3) * 16 + fr, fc);
 #pragma unroll
             for (int nt = 0; nt < 4; nt++) {
                 acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, bh[nt], acc[mt][nt], 0, 0, 0);
@@ -173,74 +188,460 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(g3k_gemm_args a) {
         }
     }
 
-    // epilogue: lane holds C rows m = base + 4 (l / 16) + i, i = 0..3, of token l % 16
-    constexpr int MO = GEGLU ? MT / 2 : MT;   // output tiles per wave along m
+    // epilogue: lane holds rows m = base + 4 (l / 16) + i, i = 0..3, of token l % 16
 #pragma unroll
-    for (int mt = 0; mt < MO; mt++)
+    for (int mt = 0; mt < MT / 2; mt++)
 #pragma unroll
         for (int nt = 0; nt < 4; nt++) {
-            const int m = m0 + (GEGLU ? wm * 64 : wm * 16 * MT) + mt * 16 + 4 * fc;
-            const int n = n0 + wn * 64 + nt * 16 + fr;
+            const int m = m0 + wm * 64 + mt * 16 + 4 * fc, n = n0 + wn * 64 + nt * 16 + fr;
             if (n >= N || m >= M) continue;   // M is a multiple of 4 (checked on the host)
-            if (GEGLU) {
-                const f32x4 g = acc[mt][nt], u = acc[mt + 4][nt];
-                uint32_t hi[4], lo[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float h = gelu_tanh(g[i]) * u[i];
-                    hi[i] = bf16_rne(h);
-                    lo[i] = bf16_rne(h - __uint_as_float(hi[i] << 16));
-                }
-                const size_t o = (size_t)n * a.ldh + m;
-                *reinterpret_cast<uint2 *>(a.h_hi + o) = make_uint2(hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16));
-                *reinterpret_cast<uint2 *>(a.h_lo + o) = make_uint2(lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16));
-            } else {
-                const f32x4 c = acc[mt][nt];
-                float *dst = a.C[m_idx] + (size_t)blockIdx.z * a.split_stride + (size_t)n * a.ldc[m_idx] + m;
-                *reinterpret_cast<float4 *>(dst) = make_float4(c[0], c[1], c[2], c[3]);
-            }
+            const f32x4 g = acc[mt][nt], u = acc[mt + 4][nt];
+            store_planes(a, n, m, gelu_tanh(g[0]) * u[0], gelu_tanh(g[1]) * u[1], gelu_tanh(g[2]) * u[2],
+                         gelu_tanh(g[3]) * u[3]);
         }
 }
 
-template <bool GEGLU, int MT>
-int launch(const g3k_gemm_args *a, hipStream_t st) {
-    constexpr int BMW = GEGLU ? 16 * MT : 32 * MT;
+// ---------------------------------------------------------------------------
+// Many tokens: 256 weight rows (GEGLU: 128 gate rows and the same 128 up
+// rows) x 128 tokens per workgroup of 8 waves, one workgroup per CU, K in
+// chunks of 64 with two chunks of LDS (2 x 64 KiB).  The eight waves are four
+// 128-row x 64-token quarters times two halves of every chunk's k values:
+// each wave reads 16 fragments for 64 MFMAs (as a 128 x 64 wave tile does
+// with 128 accumulator registers), two waves run per SIMD, and a fetch takes
+// whole 128-byte lines (8 rows x 128 B) instead of half lines (16 rows x 64
+// B, whose 64-byte requests halve what an L2 delivers).  The two k halves
+// meet through LDS at the end, each wave finishing half of its pair's tiles.
+// Split-K (ksplit) fills the chip where the tiles alone do not.
+// Against 128- and 256-row x 128-token tiles with 32-wide stages, two
+// workgroups per CU (us, Gemma3-4B shapes): 8192 tokens: Q/K/V 349 -> 338,
+// o_proj 185 -> 180, down_proj 896 -> 781; 2048: 88 -> 72, 56 -> 54, 300 ->
+// 193; 512: 53 -> 26, 22 -> 22, 79 -> 62, gate + up 136 -> 132; 256: gate +
+// up 95 -> 72.  The K loop is bound by the matrix cores at the clocks they
+// sustain and by the L2 -> LDS stream about equally (down_proj at 8192
+// without its fetches: 602 us; with a quarter of its MFMAs: 645).
+template <bool GEGLU>
+struct Pairs {
+    static constexpr int THREADS = 512, WAVES = 2;
+    static __device__ void run(const g3k_gemm_args &a);
+};
+template <bool GEGLU>
+__device__ __forceinline__ void Pairs<GEGLU>::run(const g3k_gemm_args &a) {
+    constexpr int MT = 8, NTL = 4, KC = 64;
+    constexpr int W_B = 256 * KC * 2, X_B = BN * KC * 2, STAGE_B = W_B + 2 * X_B;
+    __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE_B];
+
+    constexpr int BMW = GEGLU ? 128 : 256;               // matrix rows per workgroup
+    int bx = blockIdx.x, m_idx = 0;
+    if (!GEGLU) {
+        while (m_idx + 1 < a.n_mat && bx >= (a.M[m_idx] + BMW - 1) / BMW) {
+            bx -= (a.M[m_idx] + BMW - 1) / BMW;
+            m_idx++;
+        }
+    }
+    const int M = a.M[m_idx], K = a.K, N = a.N;
+    const int m0 = bx * BMW, n0 = blockIdx.y * BN;
+    // split z takes chunks [c0, c1) of 64 k values
+    const int chunks = (K + KC - 1) / KC;
+    const int c0 = (int)((long long)chunks * blockIdx.z / a.ksplit);
+    const int c1 = (int)((long long)chunks * (blockIdx.z + 1) / a.ksplit);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave & 1, wn = (wave >> 1) & 1, kw = wave >> 2;
+    const int fr = lane & 15, fc = lane >> 4;
+
+    // wave w fetches rows 32 w .. + 31 of the W region and of the two x
+    // planes (hi: waves 0..3, lo: 4..7), four instructions each
+    const __amdgpu_buffer_rsrc_t rw = rsrc(a.W[GEGLU ? kw : m_idx], (uint32_t)((size_t)M * K * 2));
+    const __amdgpu_buffer_rsrc_t rx = rsrc(kw ? a.x_lo : a.x_hi, (uint32_t)((size_t)N * a.ldx * 2));
+    const int dr = lane >> 3, dc = ((lane & 7) ^ dr) * 16;
+    const uint32_t wvo = (uint32_t)(m0 + (GEGLU ? wave & 3 : wave) * 32 + dr) * (uint32_t)K * 2u + dc;
+    const uint32_t xvo = (uint32_t)(n0 + (wave & 3) * 32 + dr) * (uint32_t)a.ldx * 2u + dc;
+
+    f32x4 acc[MT][NTL];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nt = 0; nt < NTL; nt++) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    auto fetch = [&](int s, int c) {
+        const uint32_t kb = (uint32_t)c * (KC * 2);
+        char *ws = smem + s * STAGE_B + wave * 4096, *xs = ws + W_B;
+#pragma unroll
+        for (int i = 0; i < 4; i++) fetch8(rw, ws + i * 1024, wvo + (uint32_t)i * (uint32_t)K * 16u, kb);
+#pragma unroll
+        for (int i = 0; i < 4; i++) fetch8(rx, xs + i * 1024, xvo + (uint32_t)i * (uint32_t)a.ldx * 16u, kb);
+    };
+    const int f = fr * 128 + (((4 * kw + fc) ^ (fr & 7)) * 16);
+    // W region row of the wave's tile mt
+    auto wrow = [&](int mt) {
+        return GEGLU ? (mt >> 2) * 128 + wm * 64 + (mt & 3) * 16 : wm * 128 + mt * 16;
+    };
+    fetch(0, c0);
+    for (int c = c0; c < c1; c++) {
+        const int s = (c - c0) & 1;
+        __syncthreads();   // chunk c has landed; the other slot is free
+        if (c + 1 < c1) fetch(s ^ 1, c + 1);
+        if (c * KC + 32 * kw >= K) continue;   // K ends with half a chunk: nothing for this half
+        const char *ws = smem + s * STAGE_B + f, *xs = smem + s * STAGE_B + W_B + wn * (64 * 128) + f;
+        bf16x8 h[NTL], l[NTL], w[2];
+#pragma unroll
+        for (int nt = 0; nt < NTL; nt++) h[nt] = *reinterpret_cast<const bf16x8 *>(xs + nt * 2048);
+        w[0] = *reinterpret_cast<const bf16x8 *>(ws + wrow(0) * 128);
+#pragma unroll
+        for (int nt = 0; nt < NTL; nt++) l[nt] = *reinterpret_cast<const bf16x8 *>(xs + X_B + nt * 2048);
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            // the next W fragment is requested ahead of this one's MFMAs
+            if (mt + 1 < MT) w[(mt + 1) & 1] = *reinterpret_cast<const bf16x8 *>(ws + wrow(mt + 1) * 128);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int nt = 0; nt < NTL; nt++)
+                acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[mt & 1], h[nt], acc[mt][nt], 0, 0, 0);
+#pragma unroll
+            for (int nt = 0; nt < NTL; nt++)
+                acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[mt & 1], l[nt], acc[mt][nt], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    __syncthreads();
+
+    // lane holds rows m = base + 4 (l / 16) + i, i = 0..3, of token l % 16
+    long long ld;
+    float *C = GEGLU ? nullptr : out_base(a, m_idx, blockIdx.z, ld);
+    f32x4 *red = reinterpret_cast<f32x4 *>(smem);   // 16 KiB per wave: its pair's half of the tiles
+    // tile t (0..3) of the half that k half hw finishes
+    auto tile = [](int hw, int t) { return GEGLU ? 4 * (t >> 1) + 2 * hw + (t & 1) : 4 * hw + t; };
+    auto hand_over = [&](int hw) {
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int nt = 0; nt < NTL; nt++) red[wave * 1024 + (t * NTL + nt) * 64 + lane] = acc[tile(hw, t)][nt];
+    };
+    if (kw) hand_over(0);
+    else hand_over(1);
+    __syncthreads();
+    auto finish = [&](int hw) {
+        const f32x4 *in = red + (wave ^ 4) * 1024 + lane;
+#pragma unroll
+        for (int t = 0; t < (GEGLU ? 2 : 4); t++) {
+            const int mt = tile(hw, t), m = m0 + (GEGLU ? wm * 64 : wm * 128) + mt * 16 + 4 * fc;
+#pragma unroll
+            for (int nt = 0; nt < NTL; nt++) {
+                const int n = n0 + wn * 64 + nt * 16 + fr;
+                f32x4 v = in[(t * NTL + nt) * 64];
+                v = hw ? v + acc[mt][nt] : acc[mt][nt] + v;
+                if (GEGLU) {
+                    const f32x4 u = acc[tile(hw, t + 2)][nt] + in[((t + 2) * NTL + nt) * 64];
+                    if (n < N && m < M)   // M is a multiple of 4 (checked on the host)
+                        store_planes(a, n, m, gelu_tanh(v[0]) * u[0], gelu_tanh(v[1]) * u[1], gelu_tanh(v[2]) * u[2],
+                                     gelu_tanh(v[3]) * u[3]);
+                } else if (n < N && m < M) {
+                    *reinterpret_cast<float4 *>(C + (size_t)n * ld + m) = make_float4(v[0], v[1], v[2], v[3]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    if (kw) finish(1);
+    else finish(0);
+}
+
+// ---------------------------------------------------------------------------
+// Few tokens: the weight stream.
+//
+// With N <= 128 tokens (a short message, a ragged tail) the projection is one
+// pass over W at the HBM rate; 128 x 128 tiles leave most CUs idle (down_proj:
+// 20 workgroups) and walk K in 0.6 us steps.  Here a workgroup of NWV waves
+// covers 16 MT NWV weight rows x 16 NTL tokens, every wave its own 16 MT rows
+// and all the tokens, and K is split until the grid fills the chip.  K moves
+// in chunks of 64: one DMA instruction takes 8 rows x 128 B (a whole line of
+// each row: 16 rows x 64 B, the MFMA operand's own shape, read W at 2.3-4.0
+// TB/s against 5.0-5.5), and DEPTH chunks are in flight in an LDS ring whose
+// barrier waits only for the oldest.  A row's eight 16-byte pieces sit at
+// c ^ (row % 8), so a fragment read (16 rows, one piece) spreads over the
+// banks.  Rows past M or N read zero; rows of a last half chunk past K hold
+// other rows' values and are not multiplied.
+// Every split writes fp32 partial products; the consumer or
+// split_reduce_kernel adds them in split order.
+template <int MT, int NTL, int DEPTH, int NWV, int OCC>
+struct Stream {
+    static constexpr int THREADS = NWV * 64, WAVES = OCC, ROWS = NWV * MT * 16, TOKENS = NTL * 16;
+    static __device__ void run(const g3k_gemm_args &a);
+};
+template <int MT, int NTL, int DEPTH, int NWV, int OCC>
+__device__ __forceinline__ void Stream<MT, NTL, DEPTH, NWV, OCC>::run(const g3k_gemm_args &a) {
+    constexpr int BM = NWV * MT * 16, KC = 64;
+    constexpr int W_B = BM * KC * 2, X_B = NTL * 16 * KC * 2;   // X_B: one plane
+    constexpr int STAGE_B = W_B + 2 * X_B;
+    constexpr int NWI = MT * 2;             // W fetches of a wave per chunk (8 rows each)
+    constexpr int NXI = NTL * 4 / NWV;      // its x_hi / x_lo fetches
+    static_assert(NTL * 4 % NWV == 0, "every wave issues the same number of fetches (counted waits)");
+    __shared__ __attribute__((aligned(1024))) char smem[DEPTH * STAGE_B];
+
+    int bx = blockIdx.x, m_idx = 0;
+    while (m_idx + 1 < a.n_mat && bx >= (a.M[m_idx] + BM - 1) / BM) {
+        bx -= (a.M[m_idx] + BM - 1) / BM;
+        m_idx++;
+    }
+    const int M = a.M[m_idx], K = a.K, N = a.N;
+    const int m0 = bx * BM, n0 = blockIdx.y * (NTL * 16);
+    // split z takes chunks [c0, c1) of 64 k values
+    const int chunks = (K + KC - 1) / KC;
+    const int c0 = (int)((long long)chunks * blockIdx.z / a.ksplit);
+    const int c1 = (int)((long long)chunks * (blockIdx.z + 1) / a.ksplit);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int fr = lane & 15, fc = lane >> 4;
+
+    const __amdgpu_buffer_rsrc_t rw = rsrc(a.W[m_idx], (uint32_t)((size_t)M * K * 2));
+    const uint32_t xbytes = (uint32_t)((size_t)N * a.ldx * 2);
+    const __amdgpu_buffer_rsrc_t rxh = rsrc(a.x_hi, xbytes), rxl = rsrc(a.x_lo, xbytes);
+    // this lane's 16 bytes of a fetch: row lane / 8, piece (lane % 8) ^ row
+    const int dr = lane >> 3, dc = ((lane & 7) ^ dr) * 16;
+    const uint32_t wbase = (uint32_t)(m0 + wave * MT * 16 + dr) * (uint32_t)K * 2u + dc;
+    const uint32_t xbase = (uint32_t)(n0 + dr) * (uint32_t)a.ldx * 2u + dc;
+
+    f32x4 acc[MT][NTL];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nt = 0; nt < NTL; nt++) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // chunk c (clamped to the split's last: the counted waits want every
+    // round to issue the same number) into ring slot s
+    auto fetch = [&](int s, int c) {
+        const uint32_t kb = (uint32_t)(c < c1 ? c : c1 - 1) * (KC * 2);
+        char *ws = smem + s * STAGE_B + wave * (MT * 2048);
+#pragma unroll
+        for (int i = 0; i < NWI; i++) fetch8(rw, ws + i * 1024, wbase + (uint32_t)i * (uint32_t)K * 16u, kb);
+        char *xs = smem + s * STAGE_B + W_B;
+#pragma unroll
+        for (int j = 0; j < NXI; j++) {
+            const int g = wave + NWV * j, r8 = g % (2 * NTL);   // 8-row group r8 of plane g / (2 NTL)
+            fetch8(g < 2 * NTL ? rxh : rxl, xs + g * 1024, xbase + (uint32_t)r8 * (uint32_t)a.ldx * 16u, kb);
+        }
+    };
+    // The ring's waits count fetches in issue order, so no round may move
+    // into another: a scheduling fence after each.
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; d++) {
+        fetch(d, c0 + d);
+        G3K_ORDER_FENCE();
+    }
+    const int f0 = fr * 128 + ((fc ^ (fr & 7)) * 16), f1 = fr * 128 + (((4 + fc) ^ (fr & 7)) * 16);
+    int slot = 0;
+    for (int c = c0; c < c1; c++) {
+        // chunk c has landed (the DEPTH - 2 rounds after it may be in flight)
+        // and every wave is done with chunk c - 1, whose slot is filled next
+        G3K_WAIT_BARRIER((DEPTH - 2) * (NWI + NXI));
+        fetch(slot == 0 ? DEPTH - 1 : slot - 1, c + DEPTH - 1);
+        G3K_ORDER_FENCE();
+        const char *ws = smem + slot * STAGE_B + wave * (MT * 2048), *xs = smem + slot * STAGE_B + W_B;
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++) {
+            if (kk == 1 && c * KC + 32 >= K) break;   // uniform: K ends with half a chunk
+            const int f = kk ? f1 : f0;
+            bf16x8 w[MT];
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) w[mt] = *reinterpret_cast<const bf16x8 *>(ws + mt * 2048 + f);
+#pragma unroll
+            for (int nt = 0; nt < NTL; nt++) {
+                const bf16x8 xh = *reinterpret_cast<const bf16x8 *>(xs + nt * 2048 + f);
+                const bf16x8 xl = *reinterpret_cast<const bf16x8 *>(xs + X_B + nt * 2048 + f);
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++)
+                    acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[mt], xh, acc[mt][nt], 0, 0, 0);
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++)
+                    acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[mt], xl, acc[mt][nt], 0, 0, 0);
+            }
+        }
+        slot = slot + 1 == DEPTH ? 0 : slot + 1;
+    }
+    // the clamped fetches past the end still write the ring
+    G3K_WAIT_VMEM();
+
+    // lane holds rows m = base + 4 (l / 16) + i, i = 0..3, of token l % 16
+    long long ld;
+    float *C = out_base(a, m_idx, blockIdx.z, ld);
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nt = 0; nt < NTL; nt++) {
+            const int m = m0 + wave * MT * 16 + mt * 16 + 4 * fc, n = n0 + nt * 16 + fr;
+            if (n >= N || m >= M) continue;   // M is a multiple of 4 (checked on the host)
+            const f32x4 c = acc[mt][nt];
+            *reinterpret_cast<float4 *>(C + (size_t)n * ld + m) = make_float4(c[0], c[1], c[2], c[3]);
+        }
+}
+
+// One launch of form F (Stream, Pairs, Gate).
+template <class F>
+__global__ __launch_bounds__(F::THREADS, F::WAVES) void gemm_kernel(g3k_gemm_args a) {
+    F::run(a);
+}
+
+// Adds the partial products a.part [ksplit][N][sum of M] in split order into
+// C (plain) or, for GEGLU, into the hi / lo planes of gelu_tanh(gate) * up.
+// One thread per four columns of one token (GEGLU: of gate and up).
+template <bool GEGLU>
+__global__ __launch_bounds__(NT) void split_reduce_kernel(g3k_gemm_args a) {
+    int ld = 0;
+    for (int j = 0; j < a.n_mat; j++) ld += a.M[j];
+    const int n = blockIdx.x, m = 4 * (blockIdx.y * NT + threadIdx.x);
+    if (m >= (GEGLU ? a.M[0] : ld)) return;
+    const size_t stride = (size_t)a.N * ld;
+    auto sum = [&](int col) {
+        const float4 *p = reinterpret_cast<const float4 *>(a.part + (size_t)n * ld + col);
+        float4 t = *p;
+#pragma unroll 8
+        for (int s = 1; s < a.ksplit; s++) {
+            const float4 v = *reinterpret_cast<const float4 *>(a.part + s * stride + (size_t)n * ld + col);
+            t = make_float4(t.x + v.x, t.y + v.y, t.z + v.z, t.w + v.w);
+        }
+        return t;
+    };
+    if (GEGLU) {
+        const float4 g = sum(m), u = sum(a.M[0] + m);
+        store_planes(a, n, m, gelu_tanh(g.x) * u.x, gelu_tanh(g.y) * u.y, gelu_tanh(g.z) * u.z, gelu_tanh(g.w) * u.w);
+        return;
+    }
+    int j = 0, col = m;
+    while (j + 1 < a.n_mat && col >= a.M[j]) col -= a.M[j++];
+    *reinterpret_cast<float4 *>(a.C[j] + (size_t)n * a.ldc[j] + col) = sum(m);
+}
+
+// Workgroups of `rows` weight rows that cover the launch's matrices.
+int row_tiles(const g3k_gemm_args *a, int rows) {
     int tiles = 0;
-    const int nm = GEGLU ? 1 : a->n_mat;
-    for (int m = 0; m < nm; m++) tiles += (a->M[m] + BMW - 1) / BMW;
-    const dim3 grid(tiles, (a->N + BN - 1) / BN, a->ksplit);
-    hipLaunchKernelGGL((gemm_kernel<GEGLU, MT>), grid, dim3(NT), 0, st, *a);
+    for (int m = 0; m < a->n_mat; m++) tiles += (a->M[m] + rows - 1) / rows;
+    return tiles;
+}
+
+int launch_reduce(const g3k_gemm_args *a, hipStream_t st) {
+    const bool geglu = a->mode == G3K_MV_GEGLU;
+    int cols = a->M[0];
+    for (int m = 1; m < a->n_mat && !geglu; m++) cols += a->M[m];
+    const dim3 grid(a->N, (cols / 4 + NT - 1) / NT);
+    if (geglu)
+        hipLaunchKernelGGL((split_reduce_kernel<true>), grid, dim3(NT), 0, st, *a);
+    else
+        hipLaunchKernelGGL((split_reduce_kernel<false>), grid, dim3(NT), 0, st, *a);
     return (int)hipGetLastError();
+}
+
+template <class F>
+int launch(const g3k_gemm_args *a, int tiles, int blocks, hipStream_t st) {
+    hipLaunchKernelGGL((gemm_kernel<F>), dim3(tiles, blocks, a->ksplit), dim3(F::THREADS), 0, st, *a);
+    return (int)hipGetLastError();
+}
+
+template <class F>
+int launch_stream(const g3k_gemm_args *a, hipStream_t st) {
+    return launch<F>(a, row_tiles(a, F::ROWS), (a->N + F::TOKENS - 1) / F::TOKENS, st);
+}
+
+int launch_form(const g3k_gemm_args *a, hipStream_t st) {
+    const int nb = (a->N + BN - 1) / BN;
+    switch (a->kind) {
+        case G3K_GEMM_WIDE:
+            if (a->N <= 32) return launch_stream<Stream<2, 2, 3, 8, 1>>(a, st);
+            if (a->N <= 64) return launch_stream<Stream<2, 4, 3, 8, 1>>(a, st);
+            return launch_stream<Stream<2, 8, 2, 8, 1>>(a, st);
+        case G3K_GEMM_NARROW:
+            if (a->N <= 16) return launch_stream<Stream<1, 1, 3, 4, 4>>(a, st);
+            if (a->N <= 32) return launch_stream<Stream<1, 2, 2, 4, 4>>(a, st);
+            return launch_stream<Stream<1, 4, 2, 4, 3>>(a, st);
+        case G3K_GEMM_GATE:
+            return launch<Gate>(a, (a->M[0] + 127) / 128, nb, st);
+        default:
+            if (a->mode == G3K_MV_GEGLU) return launch<Pairs<true>>(a, (a->M[0] + 127) / 128, nb, st);
+            return launch<Pairs<false>>(a, row_tiles(a, 256), nb, st);
+    }
 }
 
 }  // namespace
 
+// The kernel and its k splits for N tokens.
+// - Up to 128 tokens, or a product of up to 12 GFLOP issued, is a stream of W:
+//   GEGLU's many rows take 256-row workgroups, one per CU; the others 64-row
+//   ones, two per CU (one where a second launch has to add the splits and
+//   N <= 64: each split costs that launch its partial products).  Splits of
+//   less than two chunks gain nothing.
+// - Beyond, the 256 x 128 tiles: split z adds its part to the time of a round
+//   of n_cu workgroups (1.75 us per 64-wide chunk and 5 us around the K loop,
+//   measured with every CU busy) and its partial products (moved at about 8
+//   MB per us); the S with the least total is taken.
+// - GEGLU from 1536 tokens on fills several rounds of any tile, and two small
+//   workgroups per CU hide each other's epilogues: 408 us against 434 at 2048.
+extern "C" void g3k_gemm_plan(int N, int K, int n_mat, const int *M, int geglu, int consumer_adds, int n_cu, int *kind,
+                              int *ksplit) {
+    long long sum = 0, tiles64 = 0, tiles256 = 0;
+    for (int m = 0; m < n_mat; m++) {
+        sum += M[m];
+        tiles64 += (M[m] + 63) / 64;
+        tiles256 += (M[m] + 255) / 256;
+    }
+    const int chunks = (K + 63) / 64, most = chunks > 1 ? chunks / 2 : 1;
+    const int cus = n_cu > 0 ? n_cu : 256;
+    long long S = 1;
+    if (N <= 128 || (!geglu && N <= 4096 && 4.0 * N * (double)sum * K <= 12e9)) {
+        if (geglu) {
+            *kind = G3K_GEMM_WIDE;
+            S = cus / tiles256;
+        } else {
+            *kind = G3K_GEMM_NARROW;
+            const int per = N <= 16 ? 16 : N <= 32 ? 32 : 64;
+            S = (long long)cus * (!consumer_adds && N <= 64 ? 1 : 2) / (tiles64 * ((N + per - 1) / per));
+        }
+        if (S > most) S = most;
+        *ksplit = S < 1 ? 1 : (int)S;
+        return;
+    }
+    *ksplit = 1;
+    if (geglu) {
+        *kind = N >= 1536 ? G3K_GEMM_GATE : G3K_GEMM_TILE;
+        return;
+    }
+    *kind = G3K_GEMM_TILE;
+    const long long tiles = tiles256 * ((N + BN - 1) / BN);
+    double best = 0.0;
+    for (int s = 1; s <= 16 && s <= most; s++) {
+        if (s > 1 && 4.0 * s * N * (double)sum > 256e6) break;   // bounded workspace
+        double t = (double)((tiles * s + cus - 1) / cus) * (1.75 * ((chunks + s - 1) / s) + 5.0);
+        if (s > 1) t += (double)s * N * (double)sum * 8.0 / 8e6 + (consumer_adds ? 0.0 : 3.0);
+        if (s == 1 || t < best) {
+            best = t;
+            *ksplit = s;
+        }
+    }
+}
+
 extern "C" int g3k_gemm(const g3k_gemm_args *a, void *stream) {
     const bool geglu = a->mode == G3K_MV_GEGLU;
     const int S = a->ksplit;
-    if (a->N < 1 || a->K < BK || a->ldx < a->K || a->ldx % 8 || !a->x_hi || !a->x_lo)
+    if (a->N < 1 || a->K < BK || a->K % BK || a->ldx < a->K || a->ldx % 8 || !a->x_hi || !a->x_lo)
         return (int)hipErrorInvalidValue;
-    if (S < 1 || S > 16 || a->K % (BK * S) || (geglu && S != 1)) return (int)hipErrorInvalidValue;
     if (a->n_mat < 1 || a->n_mat > G3K_MATVEC_MAX || (geglu && a->n_mat != 2) || (a->mode != 0 && !geglu))
         return (int)hipErrorInvalidValue;
+    if (a->kind < G3K_GEMM_TILE || a->kind > G3K_GEMM_GATE || (a->kind == G3K_GEMM_GATE && !geglu))
+        return (int)hipErrorInvalidValue;
+    // at least one 64-wide chunk per split; the grid's y and z limits
+    const bool stream_w = a->kind == G3K_GEMM_WIDE || a->kind == G3K_GEMM_NARROW;
+    if (S < 1 || S > (a->K + 63) / 64 || S > 65535 || a->N > (stream_w ? 16 : BN) * 65535)
+        return (int)hipErrorInvalidValue;
+    // GEGLU is applied to whole sums: through part, or by an unsplit tile kernel
+    if (geglu && (stream_w ? !a->part : (S != 1 || a->part))) return (int)hipErrorInvalidValue;
     // 32-bit buffer offsets, including the rows of a last partial tile
     if ((size_t)(a->N + BN) * a->ldx * 2 >= (1ull << 32)) return (int)hipErrorInvalidValue;
-    long long tiles128 = 0;
     for (int m = 0; m < a->n_mat; m++) {
         if (a->M[m] < 4 || a->M[m] % 4 || !a->W[m] || (size_t)(a->M[m] + 256) * a->K * 2 >= (1ull << 32))
             return (int)hipErrorInvalidValue;
         if (geglu) continue;
         if (!a->C[m] || a->ldc[m] < a->M[m] || a->ldc[m] % 4) return (int)hipErrorInvalidValue;
-        if (S > 1 && a->split_stride < (long long)a->N * a->ldc[m]) return (int)hipErrorInvalidValue;
-        tiles128 += (a->M[m] + 127) / 128;
+        if (S > 1 && !a->part && a->split_stride < (long long)a->N * a->ldc[m]) return (int)hipErrorInvalidValue;
     }
+    if (geglu && (a->M[0] != a->M[1] || !a->h_hi || !a->h_lo || a->ldh < a->M[0] || a->ldh % 4))
+        return (int)hipErrorInvalidValue;
     hipStream_t st = (hipStream_t)stream;
-    if (geglu) {
-        if (a->M[0] != a->M[1] || !a->h_hi || !a->h_lo || a->ldh < a->M[0] || a->ldh % 4)
-            return (int)hipErrorInvalidValue;
-        return launch<true, 8>(a, st);
-    }
-    // 256-row tiles once they give two workgroups per CU; 128-row tiles below
-    const long long wgs256 = (tiles128 + 1) / 2 * ((a->N + BN - 1) / BN) * S;
-    return wgs256 >= 512 ? launch<false, 8>(a, st) : launch<false, 4>(a, st);
+    const int rc = launch_form(a, st);
+    return rc || !a->part ? rc : launch_reduce(a, st);
 }

@@ -1429,7 +1429,10 @@ int g3attn_matmul_bf16_device(g3attn_ctx *c, float *C, const uint16_t *W, const 
     }
     hipSetDevice(c->device);
     const size_t plane = align256((size_t)N * K * 2);
-    int rc = grow_buf(c, (float **)&c->d_big, &c->d_big_cap, 2 * plane, "matmul planes");
+    int kind, ksplit;
+    g3k_gemm_plan(N, K, 1, &M, 0, 0, c->n_cu, &kind, &ksplit);
+    const size_t part = ksplit > 1 ? (size_t)ksplit * N * M * sizeof(float) : 0;
+    int rc = grow_buf(c, (float **)&c->d_big, &c->d_big_cap, 2 * plane + part, "matmul planes");
     if (rc) return rc;
     uint16_t *xh = (uint16_t *)c->d_big, *xl = (uint16_t *)((unsigned char *)c->d_big + plane);
     g3k_rows_args r;
@@ -1452,7 +1455,9 @@ int g3attn_matmul_bf16_device(g3attn_ctx *c, float *C, const uint16_t *W, const 
     g.K = K;
     g.ldx = K;
     g.n_mat = 1;
-    g.ksplit = 1;
+    g.kind = kind;
+    g.ksplit = ksplit;
+    g.part = part ? (float *)((unsigned char *)c->d_big + 2 * plane) : NULL;
     g.W[0] = W;
     g.M[0] = M;
     g.C[0] = C;
@@ -1467,16 +1472,42 @@ int g3attn_matmul_bf16_device(g3attn_ctx *c, float *C, const uint16_t *W, const 
 /* Tokens per pass through the stack: the activations below take about 100 KiB
  * per token at Gemma3-4B shapes (0.8 GiB at 8192). */
 #define PB_CHUNK 8192
-#define PB_SPLIT_MAX 4
 
-/* k splits for a GEMM with M output rows over n tokens: the smallest power of
- * two (<= PB_SPLIT_MAX) that gives 512 workgroups of 128 x 128 (two per CU),
- * with K / S a multiple of 32. */
-static int pick_ksplit(int n, int M, int K) {
-    const long long wgs = (long long)((M + 127) / 128) * ((n + 127) / 128);
-    int S = 1;
-    while (S < PB_SPLIT_MAX && wgs * S < 512 && K % (32 * 2 * S) == 0) S *= 2;
-    return S;
+/* The projections of a chunk of n tokens, and the plan of each.  o_proj and
+ * down_proj leave their k splits to the residual step that follows. */
+enum { PB_QKV, PB_O, PB_MLP, PB_DOWN, PB_PROJS };
+typedef struct {
+    int kind, ksplit;
+} pb_plan;
+
+static void pb_plans(const g3attn_ctx *c, int n, pb_plan p[PB_PROJS]) {
+    const g3attn_config *cfg = &c->cfg;
+    const int hid = cfg->hidden_size, inter = cfg->intermediate_size;
+    const int qs = cfg->num_heads * D, ks = cfg->num_kv_heads * D;
+    const int m_qkv[3] = {qs, ks, ks}, m_mlp[2] = {inter, inter};
+    g3k_gemm_plan(n, hid, 3, m_qkv, 0, 0, c->n_cu, &p[PB_QKV].kind, &p[PB_QKV].ksplit);
+    g3k_gemm_plan(n, qs, 1, &hid, 0, 1, c->n_cu, &p[PB_O].kind, &p[PB_O].ksplit);
+    g3k_gemm_plan(n, hid, 2, m_mlp, 1, 0, c->n_cu, &p[PB_MLP].kind, &p[PB_MLP].ksplit);
+    g3k_gemm_plan(n, inter, 1, &hid, 0, 1, c->n_cu, &p[PB_DOWN].kind, &p[PB_DOWN].ksplit);
+}
+
+/* Floats of the shared product buffer t: the (partial) products of o_proj or
+ * down_proj, or the partial products of Q/K/V or of gate and up. */
+static size_t pb_products(const g3attn_ctx *c, int n) {
+    const g3attn_config *cfg = &c->cfg;
+    const size_t m[PB_PROJS] = {(size_t)(cfg->num_heads + 2 * cfg->num_kv_heads) * D, (size_t)cfg->hidden_size,
+                                2 * (size_t)cfg->intermediate_size, (size_t)cfg->hidden_size};
+    pb_plan p[PB_PROJS];
+    size_t most = 0;
+    pb_plans(c, n, p);
+    for (int i = 0; i < PB_PROJS; i++) {
+        /* Q/K/V in one split and the unsplit gate / up tiles write their outputs themselves */
+        const int own = (i == PB_QKV && p[i].ksplit == 1) ||
+                        (i == PB_MLP && p[i].kind != G3K_GEMM_WIDE && p[i].kind != G3K_GEMM_NARROW);
+        const size_t need = own ? 0 : (size_t)p[i].ksplit * n * m[i];
+        if (need > most) most = need;
+    }
+    return most;
 }
 
 typedef struct {
@@ -1484,11 +1515,14 @@ typedef struct {
     uint16_t *xh, *xl, *ah, *al, *hh, *hl;
 } pb_bufs;
 
-static int pb_layout(g3attn_ctx *c, int n, pb_bufs *b) {
+/* Buffers of chunks of up to n tokens, of which the last has `tail` (its
+ * splits may be more than the others'). */
+static int pb_layout(g3attn_ctx *c, int n, int tail, pb_bufs *b) {
     const g3attn_config *cfg = &c->cfg;
     const size_t hid = cfg->hidden_size, inter = cfg->intermediate_size;
     const size_t qs = (size_t)cfg->num_heads * D, ks = (size_t)cfg->num_kv_heads * D, N = n;
-    const size_t sz[13] = {N * hid * 4, N * qs * 4, N * ks * 4, N * ks * 4, N * qs * 4, PB_SPLIT_MAX * N * hid * 4, hid * 4,
+    const size_t t_n = pb_products(c, n), t_tail = pb_products(c, tail);
+    const size_t sz[13] = {N * hid * 4, N * qs * 4, N * ks * 4, N * ks * 4, N * qs * 4, (t_n > t_tail ? t_n : t_tail) * 4, hid * 4,
                            N * hid * 2, N * hid * 2, N * qs * 2, N * qs * 2, N * inter * 2, N * inter * 2};
     size_t total = 0;
     for (int i = 0; i < 13; i++) total += align256(sz[i]);
@@ -1522,6 +1556,8 @@ static int prefill_chunk(g3attn_ctx *c, const g3attn_weights *w, int n, int pos0
     const g3attn_config *cfg = &c->cfg;
     const int hid = cfg->hidden_size, inter = cfg->intermediate_size, L = cfg->num_layers;
     const int qs = cfg->num_heads * D, ks = cfg->num_kv_heads * D;
+    pb_plan plan[PB_PROJS];
+    pb_plans(c, n, plan);
     int rc;
     g3k_rows_args r;
     memset(&r, 0, sizeof r);
@@ -1549,7 +1585,9 @@ static int prefill_chunk(g3attn_ctx *c, const g3attn_weights *w, int n, int pos0
         g.K = hid;
         g.ldx = hid;
         g.n_mat = 3;
-        g.ksplit = 1;
+        g.kind = plan[PB_QKV].kind;
+        g.ksplit = plan[PB_QKV].ksplit;
+        g.part = g.ksplit > 1 ? b->t : NULL;
         g.W[0] = lw->q_proj;
         g.W[1] = lw->k_proj;
         g.W[2] = lw->v_proj;
@@ -1585,7 +1623,8 @@ static int prefill_chunk(g3attn_ctx *c, const g3attn_weights *w, int n, int pos0
         g.K = qs;
         g.ldx = qs;
         g.n_mat = 1;
-        g.ksplit = pick_ksplit(n, hid, qs);
+        g.kind = plan[PB_O].kind;
+        g.ksplit = plan[PB_O].ksplit;
         g.split_stride = (long long)n * hid;
         g.W[0] = lw->o_proj;
         g.M[0] = hid;
@@ -1618,7 +1657,9 @@ static int prefill_chunk(g3attn_ctx *c, const g3attn_weights *w, int n, int pos0
         g.K = hid;
         g.ldx = hid;
         g.n_mat = 2;
-        g.ksplit = 1;
+        g.kind = plan[PB_MLP].kind;
+        g.ksplit = plan[PB_MLP].ksplit;
+        g.part = g.kind == G3K_GEMM_WIDE || g.kind == G3K_GEMM_NARROW ? b->t : NULL;
         g.mode = G3K_MV_GEGLU;
         g.W[0] = lw->gate_proj;
         g.W[1] = lw->up_proj;
@@ -1635,7 +1676,8 @@ static int prefill_chunk(g3attn_ctx *c, const g3attn_weights *w, int n, int pos0
         g.K = inter;
         g.ldx = inter;
         g.n_mat = 1;
-        g.ksplit = pick_ksplit(n, hid, inter);
+        g.kind = plan[PB_DOWN].kind;
+        g.ksplit = plan[PB_DOWN].ksplit;
         g.split_stride = (long long)n * hid;
         g.W[0] = lw->down_proj;
         g.M[0] = hid;
@@ -1703,7 +1745,7 @@ int g3attn_prefill_forward_device(g3attn_ctx *c, const g3attn_weights *w, const 
     hipSetDevice(c->device);
     const int chunk = num_tokens < PB_CHUNK ? num_tokens : PB_CHUNK;
     pb_bufs b;
-    int rc = pb_layout(c, chunk, &b);
+    int rc = pb_layout(c, chunk, num_tokens % chunk ? num_tokens % chunk : chunk, &b);
     if (rc) return rc;
     if ((size_t)chunk * sizeof(int) > c->d_tok_cap) {
         HIP_TRY(hipStreamSynchronize(c->stream), "g3attn_prefill_forward_device");

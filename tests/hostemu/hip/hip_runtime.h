@@ -89,6 +89,8 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, K, int, size_t) 
 // Loads complete when issued here, so the library's explicit wait for them
 // is empty.
 #define G3K_WAIT_VMEM() ((void)0)
+#define G3K_WAIT_BARRIER(n) __syncthreads()
+#define G3K_ORDER_FENCE() ((void)0)
 // The emulated machine deals workgroup i to XCD i mod 8, as the MI355X
 // dispatcher does.
 #define G3K_XCC_ID() (blockIdx.x % 8u)

@@ -1,0 +1,89 @@
+"""The forms of the batched projection (csrc/gemm.hip) and the rule that picks
+them, at the sizes where each can go wrong: the token counts on either side of
+a form's limit, weight rows that end inside a workgroup's, K that ends with
+half a 64-wide chunk, one chunk alone, and split sums.
+
+- On the CPU the rule itself (g3k_gemm_plan): what it gives is accepted by
+  the launcher for every size the entry points take, and the split products
+  stay inside a bounded workspace.
+- On the CPU the kernels' own source on the emulated machine, and on the GPU
+  the built ones, against fp64: |C - C64| <= (2^-16 + K 2^-24) sum_k |w_k x_k|
+  per element (the hi / lo split of X, 2^-17, doubled; fp32 accumulation in
+  any order).  The GEGLU forms run in the batched prefills of
+  test_gpu_gemm.py (40 tokens) and test_gpu_model_full.py (192 and 2048).
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from helpers import DeviceBuffer, g3attn
+from test_attn_hostemu import Emu, built  # noqa: F401  (built: the emulator's build)
+
+G = g3attn()
+TILE, WIDE, NARROW, GATE = range(4)
+
+
+def plan(N, K, M, geglu=0, consumer_adds=0, n_cu=256):
+    kind, s = C.c_int(), C.c_int()
+    m = (C.c_int * len(M))(*M)
+    G.lib().g3k_gemm_plan(N, K, len(M), m, geglu, consumer_adds, n_cu, C.byref(kind), C.byref(s))
+    return kind.value, s.value
+
+
+@pytest.mark.parametrize("K", [32, 64, 96, 2048, 2592, 10240])
+def test_plan_stays_in_the_launchers_limits(K):
+    rng = np.random.default_rng(K)
+    Ns = [1, 15, 16, 17, 32, 33, 64, 65, 128, 129, 1535, 1536, 4096, 4097, 65536, 2000000]
+    for N in Ns + [int(n) for n in np.exp(rng.uniform(0, 12, 40))]:
+        for M in ([4], [64], [2560], [262208], [2048, 1024, 1024], [256, 256, 256]):
+            for adds in (0, 1):
+                kind, s = plan(N, K, M, 0, adds)
+                assert kind in (TILE, NARROW) and 1 <= s <= (K + 63) // 64, (N, M, kind, s)
+                if kind == NARROW:
+                    assert N <= 4096
+                if s > 1:
+                    assert 4 * s * N * sum(M) <= 256e6, (N, M, s)
+        kind, s = plan(N, K, [10240, 10240], 1)
+        assert 1 <= s <= (K + 63) // 64
+        assert kind == (WIDE if N <= 128 else TILE if N < 1536 else GATE)
+        assert s == 1 or kind == WIDE
+
+
+SHAPES = [(16, 64, 32), (17, 68, 96), (33, 60, 160), (65, 132, 64), (1, 4, 224)]
+
+
+@pytest.mark.parametrize("cus", [8, 256])   # few and many splits
+def test_forms_on_the_emulated_machine(built, tmp_path, cus):  # noqa: F811
+    e = Emu(tmp_path)
+    for N, M, K in SHAPES:
+        e.matmul(N, M, K)
+    e.run(HOSTEMU_CUS=cus)
+
+
+def test_many_tokens_on_the_emulated_machine(built, tmp_path):  # noqa: F811
+    """Past the weight stream's token limit: the 256 x 128 tiles, with rows
+    and tokens that end inside one and a half chunk of K at the end."""
+    assert plan(4100, 96, [4])[0] == TILE
+    e = Emu(tmp_path)
+    e.matmul(4100, 4, 96)
+    e.run()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,M,K", SHAPES + [
+    (32, 4, 64), (64, 260, 2592), (128, 2560, 2080), (129, 132, 96), (7, 8, 10240), (48, 2560, 10240),
+    (300, 2560, 10240), (1500, 1028, 2592), (4100, 4, 96), (4097, 260, 32)])
+def test_forms(N, M, K):
+    rng = np.random.default_rng(N * 7 + M * 13 + K)
+    W = ((rng.standard_normal((M, K)) / 64).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    X = rng.standard_normal((N, K)).astype(np.float32)
+    with G.Context(G.default_config(max_context=256, num_layers=6), 256) as ctx:
+        dW, dX, dC = DeviceBuffer.of(W), DeviceBuffer.of(X), DeviceBuffer(N * M * 4)
+        ctx.matmul_bf16_device(dC.ptr, dW.ptr, dX.ptr, N, M, K)
+        got = dC.download(np.float32, (N, M)).astype(np.float64)
+    W64, X64 = (W.astype(np.uint32) << 16).view(np.float32).astype(np.float64), X.astype(np.float64)
+    bound = (2.0 ** -16 + K * 2.0 ** -24) * (np.abs(X64) @ np.abs(W64).T) + 1e-30
+    ratio = float(np.max(np.abs(got - X64 @ W64.T) / bound))
+    print(f"[gemm forms] N={N} M={M} K={K} plan={plan(N, K, [M])} max err / bound = {ratio:.3f}", flush=True)
+    assert np.all(np.isfinite(got)) and ratio <= 1.0
