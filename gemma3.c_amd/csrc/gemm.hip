@@ -539,16 +539,24 @@ int launch_stream(const g3k_gemm_args *a, hipStream_t st) {
     return launch<F>(a, row_tiles(a, F::ROWS), (a->N + F::TOKENS - 1) / F::TOKENS, st);
 }
 
+// Tokens per workgroup of the 64-row stream: 48 where that covers N in as many
+// blocks as 64 does.
+int narrow_tokens(int N) {
+    return N <= 16 ? 16 : N <= 32 ? 32 : (N + 47) / 48 == (N + 63) / 64 ? 48 : 64;
+}
+
 int launch_form(const g3k_gemm_args *a, hipStream_t st) {
     const int nb = (a->N + BN - 1) / BN;
     switch (a->kind) {
         case G3K_GEMM_WIDE:
             if (a->N <= 32) return launch_stream<Stream<2, 2, 3, 8, 1>>(a, st);
             if (a->N <= 64) return launch_stream<Stream<2, 4, 3, 8, 1>>(a, st);
+            if (a->N <= 96) return launch_stream<Stream<2, 6, 2, 8, 1>>(a, st);
             return launch_stream<Stream<2, 8, 2, 8, 1>>(a, st);
         case G3K_GEMM_NARROW:
             if (a->N <= 16) return launch_stream<Stream<1, 1, 3, 4, 4>>(a, st);
             if (a->N <= 32) return launch_stream<Stream<1, 2, 2, 4, 4>>(a, st);
+            if (narrow_tokens(a->N) == 48) return launch_stream<Stream<1, 3, 2, 4, 3>>(a, st);
             return launch_stream<Stream<1, 4, 2, 4, 3>>(a, st);
         case G3K_GEMM_GATE:
             return launch<Gate>(a, (a->M[0] + 127) / 128, nb, st);
@@ -589,7 +597,7 @@ extern "C" void g3k_gemm_plan(int N, int K, int n_mat, const int *M, int geglu, 
             S = cus / tiles256;
         } else {
             *kind = G3K_GEMM_NARROW;
-            const int per = N <= 16 ? 16 : N <= 32 ? 32 : 64;
+            const int per = narrow_tokens(N);
             S = (long long)cus * (!consumer_adds && N <= 64 ? 1 : 2) / (tiles64 * ((N + per - 1) / per));
         }
         if (S > most) S = most;

@@ -150,13 +150,18 @@ extern "C" int g3k_layer_step(const g3k_layer_args *a, void *stream) {
 // ------------------------------------------------------------ batched rows
 // One workgroup of 256 threads per token row (gemma3_transformer.c:585-592,
 // 596-602, 702-724, 753-765: the reference's per-token loops of the batched
-// prefill).  Values per thread: n <= 256 * RPER.
+// prefill).  Thread i holds the PER 4-element groups i + 256 u, PER fixed per
+// row length, so every load of a row (its k splits, residual and gains) is a
+// 16-byte one requested before the first use.  A short batch is a handful of
+// rows whose cost is that one round trip (77 rows of 2560 with 6 splits: 23
+// -> 7 us against 32 masked 4-byte loads per thread and split), a long one
+// moves its rows at the HBM rate.  Rows that are not a multiple of 4 values
+// or not 16-byte aligned take 4-byte accesses in the same order.
 
 namespace {
 
 constexpr int RNT = 256;
 constexpr int RNW = RNT / 64;
-constexpr int RPER = G3K_LAYER_MAX_HIDDEN / RNT;
 
 __device__ __forceinline__ float rblock_sum(float v, float *red) {
     v = wave_sum(v);
@@ -175,92 +180,170 @@ __device__ __forceinline__ uint32_t rne16(float f) {
     return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
 }
 
-// y = v * r * gain (gain 1 where w is NULL) as bf16 hi / lo planes
-__device__ __forceinline__ void store_split(const g3k_rows_args &a, int row, const float (&v)[RPER], float r,
-                                            const uint16_t *w) {
-    uint16_t *yh = a.y_hi + (size_t)row * a.ldy, *yl = a.y_lo + (size_t)row * a.ldy;
-#pragma unroll
-    for (int u = 0; u < RPER; u++) {
-        const int i = threadIdx.x + RNT * u;
-        if (i < a.n) {
-            const float y = w ? v[u] * r * (1.0f + bf16f(w[i])) : v[u];
-            const uint32_t hi = rne16(y);
-            yh[i] = (uint16_t)hi;
-            yl[i] = (uint16_t)rne16(y - __uint_as_float(hi << 16));
-        }
+// Group g (values 4 g .. 4 g + 3) of a row of n values; past the end 0.
+template <bool VEC>
+__device__ __forceinline__ float4 load4(const float *p, int g, int n) {
+    const int i = 4 * g;
+    if (VEC) {
+        const float4 v = reinterpret_cast<const float4 *>(p)[i < n ? g : 0];
+        return i < n ? v : make_float4(0.f, 0.f, 0.f, 0.f);
     }
+    return make_float4(i < n ? p[i] : 0.f, i + 1 < n ? p[i + 1] : 0.f, i + 2 < n ? p[i + 2] : 0.f,
+                       i + 3 < n ? p[i + 3] : 0.f);
 }
 
+template <bool VEC>
+__device__ __forceinline__ void store4(float *p, int g, int n, float4 v) {
+    const int i = 4 * g;
+    if (VEC) {
+        if (i < n) reinterpret_cast<float4 *>(p)[g] = v;
+        return;
+    }
+    if (i < n) p[i] = v.x;
+    if (i + 1 < n) p[i + 1] = v.y;
+    if (i + 2 < n) p[i + 2] = v.z;
+    if (i + 3 < n) p[i + 3] = v.w;
+}
+
+// Four bf16 values; al8: the array is 8-byte aligned (uniform).
+template <bool VEC>
+__device__ __forceinline__ float4 load_bf4(const uint16_t *p, int g, int n, bool al8) {
+    const int i = 4 * g;
+    if (VEC && al8) {
+        const uint2 w = reinterpret_cast<const uint2 *>(p)[i < n ? g : 0];
+        const float4 v = make_float4(bf16f(w.x & 0xffff), bf16f(w.x >> 16), bf16f(w.y & 0xffff), bf16f(w.y >> 16));
+        return i < n ? v : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    return make_float4(i < n ? bf16f(p[i]) : 0.f, i + 1 < n ? bf16f(p[i + 1]) : 0.f, i + 2 < n ? bf16f(p[i + 2]) : 0.f,
+                       i + 3 < n ? bf16f(p[i + 3]) : 0.f);
+}
+
+__device__ __forceinline__ bool aligned8(const void *p) { return ((uintptr_t)p & 7) == 0; }
+
+// y as bf16 hi / lo planes
+template <bool VEC>
+__device__ __forceinline__ void store_split(const g3k_rows_args &a, int row, int g, float4 y) {
+    const float v[4] = {y.x, y.y, y.z, y.w};
+    uint32_t hi[4], lo[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        hi[j] = rne16(v[j]);
+        lo[j] = rne16(v[j] - __uint_as_float(hi[j] << 16));
+    }
+    uint16_t *yh = a.y_hi + (size_t)row * a.ldy + 4 * g, *yl = a.y_lo + (size_t)row * a.ldy + 4 * g;
+    if (VEC) {
+        if (4 * g >= a.n) return;
+        *reinterpret_cast<uint2 *>(yh) = make_uint2(hi[0] | hi[1] << 16, hi[2] | hi[3] << 16);
+        *reinterpret_cast<uint2 *>(yl) = make_uint2(lo[0] | lo[1] << 16, lo[2] | lo[3] << 16);
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        if (4 * g + j < a.n) {
+            yh[j] = (uint16_t)hi[j];
+            yl[j] = (uint16_t)lo[j];
+        }
+}
+
+__device__ __forceinline__ float4 scale4(float4 v, float r, float4 w) {
+    return make_float4(v.x * r * (1.0f + w.x), v.y * r * (1.0f + w.y), v.z * r * (1.0f + w.z), v.w * r * (1.0f + w.w));
+}
+__device__ __forceinline__ float4 add4(float4 a, float4 b) {
+    return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+}
+
+// 1 / sqrtf(mean(v^2) + eps) of the row held PER groups per thread (0 past its end)
+template <int PER>
+__device__ __forceinline__ float row_scale(const float4 (&v)[PER], int n, float eps, float *red) {
+    float ss = 0.f;
+#pragma unroll
+    for (int u = 0; u < PER; u++) ss += v[u].x * v[u].x + v[u].y * v[u].y + v[u].z * v[u].z + v[u].w * v[u].w;
+    return 1.0f / sqrtf(rblock_sum(ss, red) / (float)n + eps);
+}
+
+template <int PER, bool VEC>
 __global__ __launch_bounds__(RNT) void rows_kernel(g3k_rows_args a) {
     __shared__ float red[RNW];
-    const int row = blockIdx.x, n = a.n;
-    float v[RPER];
+    const int row = blockIdx.x, n = a.n, tid = threadIdx.x;
     if (a.op == G3K_ROWS_SPLIT) {   // elementwise: any row length
         const float *t = a.t + (size_t)row * a.ldt;
-        uint16_t *yh = a.y_hi + (size_t)row * a.ldy, *yl = a.y_lo + (size_t)row * a.ldy;
-        for (int i = threadIdx.x; i < n; i += RNT) {
-            const float y = t[i];
-            const uint32_t hi = rne16(y);
-            yh[i] = (uint16_t)hi;
-            yl[i] = (uint16_t)rne16(y - __uint_as_float(hi << 16));
-        }
+        for (int g = tid; 4 * g < n; g += RNT) store_split<VEC>(a, row, g, load4<VEC>(t, g, n));
         return;
     }
     float *x = a.x + (size_t)row * n;
+    float4 v[PER], gn[PER];
+    const bool next = a.w_next && a.y_hi;
+    if (next) {
+#pragma unroll
+        for (int u = 0; u < PER; u++) gn[u] = load_bf4<VEC>(a.w_next, tid + RNT * u, n, aligned8(a.w_next));
+    }
     if (a.op == G3K_ROWS_EMBED) {
         const float scale = sqrtf((float)n);
         const uint16_t *e = a.embed + (size_t)a.tokens[row] * n;
 #pragma unroll
-        for (int u = 0; u < RPER; u++) {
-            const int i = threadIdx.x + RNT * u;
-            v[u] = i < n ? bf16f(e[i]) * scale : 0.f;
-            if (i < n) x[i] = v[u];
+        for (int u = 0; u < PER; u++) {
+            const float4 b = load_bf4<VEC>(e, tid + RNT * u, n, aligned8(e));
+            v[u] = make_float4(b.x * scale, b.y * scale, b.z * scale, b.w * scale);
+            store4<VEC>(x, tid + RNT * u, n, v[u]);
         }
     } else {
         const float *t = a.t + (size_t)row * a.ldt;
-        float tv[RPER];
+        float4 tv[PER], gp[PER];
 #pragma unroll
-        for (int u = 0; u < RPER; u++) {
-            const int i = threadIdx.x + RNT * u;
-            tv[u] = i < n ? t[i] : 0.f;
-            v[u] = i < n ? x[i] : 0.f;
-        }
-        for (int s = 1; s < a.nsplit; s++) {   // the k splits of the producing GEMM, in order
-            const float *ts = t + (size_t)s * a.split_stride;
-#pragma unroll
-            for (int u = 0; u < RPER; u++) {
-                const int i = threadIdx.x + RNT * u;
-                if (i < n) tv[u] += ts[i];
-            }
+        for (int u = 0; u < PER; u++) {
+            tv[u] = load4<VEC>(t, tid + RNT * u, n);
+            v[u] = load4<VEC>(x, tid + RNT * u, n);
         }
         if (a.w_post) {
-            float ss = 0.f;
 #pragma unroll
-            for (int u = 0; u < RPER; u++) ss += tv[u] * tv[u];
-            const float r = 1.0f / sqrtf(rblock_sum(ss, red) / (float)n + a.eps);
+            for (int u = 0; u < PER; u++) gp[u] = load_bf4<VEC>(a.w_post, tid + RNT * u, n, aligned8(a.w_post));
+        }
+        // the k splits of the producing GEMM, added in order, four at a time
+        for (int s = 1; s < a.nsplit; s += 4) {
+            float4 p[4][PER];
 #pragma unroll
-            for (int u = 0; u < RPER; u++) {
-                const int i = threadIdx.x + RNT * u;
-                tv[u] = i < n ? tv[u] * r * (1.0f + bf16f(a.w_post[i])) : 0.f;
+            for (int j = 0; j < 4; j++) {
+                const float *ts = t + (size_t)min(s + j, a.nsplit - 1) * a.split_stride;
+#pragma unroll
+                for (int u = 0; u < PER; u++) p[j][u] = load4<VEC>(ts, tid + RNT * u, n);
             }
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (s + j < a.nsplit) {
+#pragma unroll
+                    for (int u = 0; u < PER; u++) tv[u] = add4(tv[u], p[j][u]);
+                }
+        }
+        if (a.w_post) {
+            const float r = row_scale<PER>(tv, n, a.eps, red);
+#pragma unroll
+            for (int u = 0; u < PER; u++) tv[u] = scale4(tv[u], r, gp[u]);   // 0 past n
         }
 #pragma unroll
-        for (int u = 0; u < RPER; u++) {
-            const int i = threadIdx.x + RNT * u;
-            v[u] = v[u] + tv[u];
-            if (i < n) x[i] = v[u];
+        for (int u = 0; u < PER; u++) {
+            v[u] = add4(v[u], tv[u]);
+            store4<VEC>(x, tid + RNT * u, n, v[u]);
         }
         if (!a.y_hi) return;   // uniform
     }
-    float r = 1.f;
-    if (a.w_next) {
-        float ss = 0.f;
+    if (next) {
+        const float r = row_scale<PER>(v, n, a.eps, red);
 #pragma unroll
-        for (int u = 0; u < RPER; u++) ss += v[u] * v[u];
-        r = 1.0f / sqrtf(rblock_sum(ss, red) / (float)n + a.eps);
+        for (int u = 0; u < PER; u++) v[u] = scale4(v[u], r, gn[u]);
     }
-    store_split(a, row, v, r, a.w_next);
+#pragma unroll
+    for (int u = 0; u < PER; u++) store_split<VEC>(a, row, tid + RNT * u, v[u]);
 }
+
+template <int PER>
+void launch_rows(const g3k_rows_args *a, bool vec, hipStream_t st) {
+    if (vec)
+        hipLaunchKernelGGL((rows_kernel<PER, true>), dim3(a->rows), dim3(RNT), 0, st, *a);
+    else
+        hipLaunchKernelGGL((rows_kernel<PER, false>), dim3(a->rows), dim3(RNT), 0, st, *a);
+}
+
+bool aligned(const void *p, size_t b) { return ((uintptr_t)p & (b - 1)) == 0; }
 
 }  // namespace
 
@@ -283,6 +366,18 @@ extern "C" int g3k_rows(const g3k_rows_args *a, void *stream) {
         default:
             return (int)hipErrorInvalidValue;
     }
-    hipLaunchKernelGGL(rows_kernel, dim3(a->rows), dim3(RNT), 0, (hipStream_t)stream, *a);
+    const bool has_x = a->op != G3K_ROWS_SPLIT, has_t = a->op != G3K_ROWS_EMBED;
+    const bool vec = a->n % 4 == 0 && (!has_x || aligned(a->x, 16)) &&
+                     (!has_t || (aligned(a->t, 16) && a->ldt % 4 == 0 && (a->nsplit < 2 || a->split_stride % 4 == 0))) &&
+                     (!a->y_hi || (aligned(a->y_hi, 8) && aligned(a->y_lo, 8) && a->ldy % 4 == 0));
+    hipStream_t st = (hipStream_t)stream;
+    const int per = a->op == G3K_ROWS_SPLIT ? 1 : (a->n + 4 * RNT - 1) / (4 * RNT);
+    switch (per) {
+        case 1: launch_rows<1>(a, vec, st); break;
+        case 2: launch_rows<2>(a, vec, st); break;
+        case 3: launch_rows<3>(a, vec, st); break;
+        case 4: launch_rows<4>(a, vec, st); break;
+        default: launch_rows<8>(a, vec, st); break;
+    }
     return (int)hipGetLastError();
 }

@@ -87,3 +87,54 @@ def test_forms(N, M, K):
     ratio = float(np.max(np.abs(got - X64 @ W64.T) / bound))
     print(f"[gemm forms] N={N} M={M} K={K} plan={plan(N, K, [M])} max err / bound = {ratio:.3f}", flush=True)
     assert np.all(np.isfinite(got)) and ratio <= 1.0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K", [(3, 96), (70, 2592)])
+def test_unaligned_activations(N, K):
+    """X that is only 4-byte aligned (a slice of a caller's buffer): the split
+    into planes falls back to 4-byte loads."""
+    rng = np.random.default_rng(N + K)
+    W = ((rng.standard_normal((64, K)) / 64).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    X = rng.standard_normal((N, K)).astype(np.float32)
+    with G.Context(G.default_config(max_context=256, num_layers=6), 256) as ctx:
+        dW, dC = DeviceBuffer.of(W), DeviceBuffer(N * 64 * 4)
+        dX = DeviceBuffer.of(np.concatenate([np.zeros(1, np.float32), X.reshape(-1)]))
+        ctx.matmul_bf16_device(dC.ptr, dW.ptr, dX.ptr + 4, N, 64, K)
+        got = dC.download(np.float32, (N, 64)).astype(np.float64)
+    W64, X64 = (W.astype(np.uint32) << 16).view(np.float32).astype(np.float64), X.astype(np.float64)
+    bound = (2.0 ** -16 + K * 2.0 ** -24) * (np.abs(X64) @ np.abs(W64).T)
+    assert np.all(np.abs(got - X64 @ W64.T) <= bound)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hidden", [32, 1056, 2080, 3104, 8192])
+def test_row_lengths(hidden):
+    """The per-row norm and residual steps at each row length class (1, 2, 3,
+    4 and 8 groups of four values per thread): a one-layer batched prefill
+    against the token forward over the same tokens, at the 1e-3 x RMS bar of
+    the whole-model test (x as two bf16 planes against fp32)."""
+    n, inter, vocab = 17, 64, 96
+    rng = np.random.default_rng(hidden)
+
+    def w(*shape, scale):
+        return ((rng.standard_normal(shape) * scale).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+
+    s = 1 / np.sqrt(hidden)
+    layer = dict(input_layernorm=w(hidden, scale=0.1), q_proj=w(2048, hidden, scale=s), k_proj=w(1024, hidden, scale=s),
+                 v_proj=w(1024, hidden, scale=s), o_proj=w(hidden, 2048, scale=0.02), q_norm=w(256, scale=0.1),
+                 k_norm=w(256, scale=0.1), post_attention_layernorm=w(hidden, scale=0.1),
+                 gate_proj=w(inter, hidden, scale=s), up_proj=w(inter, hidden, scale=s),
+                 down_proj=w(hidden, inter, scale=0.1), pre_feedforward_layernorm=w(hidden, scale=0.1),
+                 post_feedforward_layernorm=w(hidden, scale=0.1))
+    tokens = rng.integers(0, vocab, n).astype(np.int32)
+    HW, keep = G.host_weights(w(vocab, hidden, scale=1.0), [layer], w(hidden, scale=0.1))
+    cfg = G.default_config(num_layers=1, hidden_size=hidden, intermediate_size=inter, vocab_size=vocab, max_context=64)
+    with G.Context(cfg, 64) as ctx:
+        ctx.upload_weights(HW)
+        got = ctx.prefill_tokens(tokens)
+        for i, t in enumerate(tokens):
+            want = ctx.forward_token(t, i)
+    e = float(np.max(np.abs(got - want)) / np.sqrt(np.mean(want.astype(np.float64) ** 2)))
+    print(f"[rows hidden={hidden}] batched vs token loop {e:.2e}", flush=True)
+    assert e <= 1e-3
