@@ -204,6 +204,9 @@ typedef struct {
     const int *v_lo_flag;
     int epoch;
     float *out;
+    /* when set, the output goes to bf16 planes [n][H_q][D] instead of out:
+     * out_hi = bf16(o), out_lo = bf16(o - out_hi), a projection's operand */
+    uint16_t *out_hi, *out_lo;
     long long ldk;
     int n, hist, nk, window;  /* window: INT_MAX / 2 for global layers */
     int n_kv_heads, group;
@@ -211,14 +214,15 @@ typedef struct {
     int queries_per_wave;     /* 16 (8 waves, 2 per SIMD) or 32 (4 waves, 1 per SIMD) */
     int schedule;             /* 16 queries per wave: 0 = all waves in phase, 1 = SIMD pairs in opposite phase */
     void *ev0, *ev1;          /* hipEvent_t: begin / end of prefill_kernel's dispatch, or NULL */
-    /* Key splits (1, 2 or 4).  With S > 1 every (query block, KV head) runs as
+    /* Key splits (1, 2, 4, 8 or 16).  With S > 1 every (query block, KV head) runs as
      * S workgroups over consecutive parts of its key tiles; each writes its
      * unnormalised O and (max, sum) per query row to part_o [S][n][H_q][D]
      * and part_ml [S][n][H_q][2], then counts itself in arrive[qb * H_kv +
      * kvh] (an atomic increment that wraps to 0 after S arrivals, so the
      * counters start every call at zero).  The last of the S workgroups to
      * arrive merges the S parts into out, in split order (deterministic).
-     * arrive holds G3K_PREFILL_ARRIVE(max_n, H_kv) zeroed counters. */
+     * arrive holds G3K_PREFILL_ARRIVE(max_n, H_kv) zeroed counters.  S > 4
+     * (few query blocks over many keys) is merged by a second launch. */
     int ksplit;
     float *part_o, *part_ml;
     unsigned *arrive;

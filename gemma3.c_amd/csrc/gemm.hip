@@ -554,9 +554,9 @@ int launch_form(const g3k_gemm_args *a, hipStream_t st) {
             if (a->N <= 96) return launch_stream<Stream<2, 6, 2, 8, 1>>(a, st);
             return launch_stream<Stream<2, 8, 2, 8, 1>>(a, st);
         case G3K_GEMM_NARROW:
-            if (a->N <= 16) return launch_stream<Stream<1, 1, 3, 4, 4>>(a, st);
-            if (a->N <= 32) return launch_stream<Stream<1, 2, 2, 4, 4>>(a, st);
-            if (narrow_tokens(a->N) == 48) return launch_stream<Stream<1, 3, 2, 4, 3>>(a, st);
+            if (a->N <= 16) return launch_stream<Stream<1, 1, 5, 4, 2>>(a, st);
+            if (a->N <= 32) return launch_stream<Stream<1, 2, 3, 4, 2>>(a, st);
+            if (narrow_tokens(a->N) == 48) return launch_stream<Stream<1, 3, 3, 4, 2>>(a, st);
             return launch_stream<Stream<1, 4, 2, 4, 3>>(a, st);
         case G3K_GEMM_GATE:
             return launch<Gate>(a, (a->M[0] + 127) / 128, nb, st);
@@ -572,7 +572,7 @@ int launch_form(const g3k_gemm_args *a, hipStream_t st) {
 // - Up to 128 tokens, or a product of up to 12 GFLOP issued, is a stream of W:
 //   GEGLU's many rows take 256-row workgroups, one per CU; the others 64-row
 //   ones, two per CU (one where a second launch has to add the splits and
-//   N <= 64: each split costs that launch its partial products).  Splits of
+//   N <= 96: each split costs that launch its partial products).  Splits of
 //   less than two chunks gain nothing.
 // - Beyond, the 256 x 128 tiles: split z adds its part to the time of a round
 //   of n_cu workgroups (1.75 us per 64-wide chunk and 5 us around the K loop,
@@ -598,7 +598,7 @@ extern "C" void g3k_gemm_plan(int N, int K, int n_mat, const int *M, int geglu, 
         } else {
             *kind = G3K_GEMM_NARROW;
             const int per = narrow_tokens(N);
-            S = (long long)cus * (!consumer_adds && N <= 64 ? 1 : 2) / (tiles64 * ((N + per - 1) / per));
+            S = (long long)cus * (!consumer_adds && N <= 96 ? 1 : 2) / (tiles64 * ((N + per - 1) / per));
         }
         if (S > most) S = most;
         *ksplit = S < 1 ? 1 : (int)S;

@@ -77,6 +77,7 @@ constexpr int LDS_KS0 = LDS_BYTES;           // fp8 cross policy: key-scale ring
 constexpr int KS_SLOT = 256;                 // one tile's 32 scale bytes (a 256-byte fetch)
 constexpr int LDS_BYTES_X8 = LDS_KS0 + 2 * KS_SLOT;
 constexpr float NEG_BIG = -1.0e30f;
+constexpr int PREFILL_MERGE_IN = 4;           // most key splits merged inside the kernel
 constexpr float LAZY = 8.0f;                 // log2 headroom of the lazy max
 #ifndef G3K_KPF
 #define G3K_KPF 1                            // K fragment prefetch depth (d-steps)
@@ -526,6 +527,21 @@ __device__ __forceinline__ void load_queries(half8 (&qh)[8], u32x4 (&qlo)[8], in
     }
 }
 
+// Four output values at element e of [n][H_q][D]: fp32, or the bf16 hi / lo
+// planes that o_proj reads (the same split as its own step would make of the
+// fp32 values, without their round trip through memory).
+__device__ __forceinline__ void store_out(const g3k_prefill_args &p, size_t e, float a, float b, float c, float d) {
+    if (!p.out_hi) {
+        *reinterpret_cast<float4 *>(p.out + e) = make_float4(a, b, c, d);
+        return;
+    }
+    const uint32_t h0 = bf16_pair(a, b), h1 = bf16_pair(c, d);
+    *reinterpret_cast<uint2 *>(p.out_hi + e) = make_uint2(h0, h1);
+    *reinterpret_cast<uint2 *>(p.out_lo + e) =
+        make_uint2(bf16_pair(a - __uint_as_float(h0 << 16), b - __uint_as_float(h0 & 0xffff0000u)),
+                   bf16_pair(c - __uint_as_float(h1 << 16), d - __uint_as_float(h1 & 0xffff0000u)));
+}
+
 // One workgroup's attention: 8 / NQB waves, each owning NQB blocks of 16
 // queries of one head over the full head dim.  VLO adds the P_hi.V_lo pass;
 // X8 selects the fp8 cross policy of the scores (staged key rows in that
@@ -824,6 +840,7 @@ __device__ __forceinline__ void attend(const g3k_prefill_args &p, unsigned char 
                 __hip_atomic_store(ml + 1, lt[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
+        if (S > PREFILL_MERGE_IN) return;   // uniform: merged by prefill_merge_kernel
         // Every part store of the wave has completed (vmcnt counts stores on
         // this family) before the block's arrival is counted; the counter
         // wraps to 0 on the S-th arrival, ready for the next call.  The
@@ -842,11 +859,11 @@ __device__ __forceinline__ void attend(const g3k_prefill_args &p, unsigned char 
             const int tok = tok0 + 16 * b + ln;
             if (tok >= p.n) continue;
             const unsigned voff = (unsigned)((((tok - qb * PB) * hq + qhead) * D + 4 * g) * 4);
-            // S <= 4: fixed trip counts keep ms / ls in registers
-            float ms[4], ls[4];
+            // S <= PREFILL_MERGE_IN: fixed trip counts keep ms / ls in registers
+            float ms[PREFILL_MERGE_IN], ls[PREFILL_MERGE_IN];
             float M = NEG_BIG;
 #pragma unroll
-            for (int sp = 0; sp < 4; sp++) {
+            for (int sp = 0; sp < PREFILL_MERGE_IN; sp++) {
                 if (sp >= S) break;
                 if (sp == split) {
                     ms[sp] = m_ref[b];
@@ -863,7 +880,7 @@ __device__ __forceinline__ void attend(const g3k_prefill_args &p, unsigned char 
 #pragma unroll
             for (int mt = 0; mt < 16; mt++) A[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int sp = 0; sp < 4; sp++) {
+            for (int sp = 0; sp < PREFILL_MERGE_IN; sp++) {
                 if (sp >= S) break;
                 const float f = fast_exp2(ms[sp] - M);
                 L += ls[sp] * f;
@@ -878,11 +895,10 @@ __device__ __forceinline__ void attend(const g3k_prefill_args &p, unsigned char 
                 }
             }
             const float inv = 1.0f / L;
-            float *orow = p.out + ((size_t)tok * hq + qhead) * D + 4 * g;
+            const size_t e = ((size_t)tok * hq + qhead) * D + 4 * g;
 #pragma unroll
             for (int mt = 0; mt < 16; mt++)
-                *reinterpret_cast<float4 *>(orow + 16 * mt) =
-                    make_float4(A[mt][0] * inv, A[mt][1] * inv, A[mt][2] * inv, A[mt][3] * inv);
+                store_out(p, e + 16 * mt, A[mt][0] * inv, A[mt][1] * inv, A[mt][2] * inv, A[mt][3] * inv);
         }
         return;
     }
@@ -892,11 +908,10 @@ __device__ __forceinline__ void attend(const g3k_prefill_args &p, unsigned char 
         const float inv = 1.0f / col4_sum(l_sum[b]);   // all lanes active here
         const int tok = tok0 + 16 * b + ln;
         if (tok >= p.n) continue;
-        float *orow = p.out + ((size_t)tok * p.n_kv_heads * G + qhead) * D + 4 * g;
+        const size_t e = ((size_t)tok * p.n_kv_heads * G + qhead) * D + 4 * g;
 #pragma unroll
         for (int mt = 0; mt < 16; mt++)
-            *reinterpret_cast<float4 *>(orow + 16 * mt) =
-                make_float4(o[b][mt][0] * inv, o[b][mt][1] * inv, o[b][mt][2] * inv, o[b][mt][3] * inv);
+            store_out(p, e + 16 * mt, o[b][mt][0] * inv, o[b][mt][1] * inv, o[b][mt][2] * inv, o[b][mt][3] * inv);
     }
 }
 
@@ -911,6 +926,43 @@ __global__ __launch_bounds__(512 / NQB, 1) void prefill_kernel(g3k_prefill_args 
         attend<G, NQB, false, X8>(p, smem);
 }
 
+// The parts of S > PREFILL_MERGE_IN key splits -> out, in split order.  A
+// block's last workgroup would read all S parts alone (15 x 128 KiB at S =
+// 16, ~18 us on one CU); here every (token, query head) row is one wave, lane
+// l holding dims 4 l .. + 3, and the splits' parts arrive eight at a time.
+__global__ __launch_bounds__(NT) void prefill_merge_kernel(g3k_prefill_args p) {
+    const int hq = p.n_kv_heads * p.group, S = p.ksplit;
+    const long long row = ((long long)blockIdx.x * NT + threadIdx.x) >> 6, rows = (long long)p.n * hq;
+    if (row >= rows) return;   // uniform per wave
+    const int lane = threadIdx.x & 63;
+    // lane s: split s's max and sum
+    float m = NEG_BIG, l = 0.f;
+    if (lane < S) {
+        const float2 ml = reinterpret_cast<const float2 *>(p.part_ml)[(size_t)lane * rows + row];
+        m = ml.x;
+        l = ml.y;
+    }
+    const float f = fast_exp2(m - wave_max(m));
+    const float inv = 1.0f / wave_sum(l * f);
+    const float4 *part = reinterpret_cast<const float4 *>(p.part_o) + (size_t)row * (D / 4) + lane;
+    const size_t stride = (size_t)rows * (D / 4);
+    float a[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < S; s += 8) {   // S is 8 or 16
+        float4 v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = part[(size_t)(s + j) * stride];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const float w = __shfl(f, s + j);
+            a[0] += v[j].x * w;
+            a[1] += v[j].y * w;
+            a[2] += v[j].z * w;
+            a[3] += v[j].w * w;
+        }
+    }
+    store_out(p, (size_t)row * D + 4 * lane, a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv);
+}
+
 template <int G, int NQB>
 hipError_t launch_prefill(const g3k_prefill_args *a, hipStream_t st) {
     constexpr int PB = 16 * NQB * ((8 / NQB) / G);
@@ -923,6 +975,10 @@ hipError_t launch_prefill(const g3k_prefill_args *a, hipStream_t st) {
     else
         hipExtLaunchKernelGGL((prefill_kernel<G, NQB, false>), grid, dim3(512 / NQB), 0, st, (hipEvent_t)a->ev0,
                               (hipEvent_t)a->ev1, 0, *a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || a->ksplit <= PREFILL_MERGE_IN) return e;
+    const long long waves = (long long)a->n * a->n_kv_heads * a->group;
+    hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(NT), 0, st, *a);
     return hipGetLastError();
 }
 
@@ -969,7 +1025,7 @@ extern "C" int g3k_prefill(const g3k_prefill_args *a, void *stream) {
     if (a->ldk % 64 || a->ldk > (1LL << 20) || a->nk > a->ldk || a->hist + a->n != a->nk ||
         a->window < 1 || !a->v_lo_flag)
         return (int)hipErrorInvalidValue;
-    if ((a->ksplit != 1 && a->ksplit != 2 && a->ksplit != 4) ||
+    if ((a->ksplit != 1 && a->ksplit != 2 && a->ksplit != 4 && a->ksplit != 8 && a->ksplit != 16) || (!a->out_hi != !a->out_lo) ||
         (a->ksplit > 1 && (!a->part_o || !a->part_ml || !a->arrive)))
         return (int)hipErrorInvalidValue;
     hipStream_t st = (hipStream_t)stream;

@@ -154,7 +154,7 @@ struct g3attn_ctx {
     int min_rows;   /* smallest heuristic split */
     int prefill_qpw; /* prefill queries per wave: 16 or 32 (G3ATTN_PREFILL_QPW) */
     int prefill_sched; /* prefill phase schedule 0 / 1 (G3ATTN_PREFILL_SCHED) */
-    int prefill_ksplit; /* G3ATTN_PREFILL_SPLITS: 1, 2 or 4 key splits for every prefill; 0 = the
+    int prefill_ksplit; /* G3ATTN_PREFILL_SPLITS: 1, 2, 4, 8 or 16 key splits for every prefill; 0 = the
                          * makespan model (prefill_splits) */
     int prefill_x8;    /* prefill scores: 1 = fp16 hi + fp8 cross terms (default), 0 = three
                         * fp16 passes (G3ATTN_PREFILL_QK=exact) */
@@ -367,7 +367,7 @@ g3attn_ctx *g3attn_create(const g3attn_config *cfg, int max_context,
         c->prefill_x8 = !(qk && strcmp(qk, "exact") == 0);
         const char *ks = getenv("G3ATTN_PREFILL_SPLITS");
         const int ksv = ks ? atoi(ks) : 0;
-        c->prefill_ksplit = (ksv == 1 || ksv == 2 || ksv == 4) ? ksv : 0;
+        c->prefill_ksplit = (ksv == 1 || ksv == 2 || ksv == 4 || ksv == 8 || ksv == 16) ? ksv : 0;
         const char *xm = getenv("G3ATTN_DECODE_XMERGE");
         c->xmerge = xm ? atoi(xm) : 1;
         const char *nt = getenv("G3ATTN_DECODE_NT");
@@ -855,10 +855,10 @@ static int grow_pf(g3attn_ctx *c, size_t bytes) {
     return G3_OK;
 }
 
-/* Key splits S (1, 2 or 4) of a prefill call.  A workgroup walks the key
+/* Key splits S (1, 2, 4, 8 or 16) of a prefill call.  A workgroup walks the key
  * tiles of one query block (pb tokens) of one KV head; with S > 1 each
  * block's tiles are dealt to S workgroups, and the last of them to finish
- * merges their parts (inside the kernel).  S minimises a makespan model
+ * merges their parts (inside the kernel; beyond 4 splits a second launch does).  S minimises a makespan model
  * measured on MI355X:
  * - a tile step costs ~2.2 us, and a workgroup ~12 us more: its prologue
  *   (queries, RoPE rows and the first K / V tiles, read while every CU does
@@ -866,8 +866,11 @@ static int grow_pf(g3attn_ctx *c, size_t bytes) {
  * - one workgroup runs per CU (its LDS), and the longest block's part sets a
  *   floor (a 4096-token global prefill unsplit: 128 tiles on one CU while
  *   the average is 65);
- * - the parts and the merge move about (S + 1) n H_q 256 floats at ~5 TB/s.
- * Each split keeps at least 4 tiles. */
+ * - the parts and the merge move about (S + 1) n H_q 256 floats at ~5 TB/s,
+ *   and the second launch of S > 4 takes ~4 us more.
+ * Each split keeps at least 4 tiles.  More than 4 splits are what a follow-up
+ * message over a long history takes: 333 tokens at position 2500, one KV
+ * head, are 11 query blocks of 85 tiles each (S = 4: 90 us, 16: 46). */
 static int prefill_splits(int n, int hist, int nk, int window, int pb, int n_kv, int n_q, int n_cu) {
     const int nb = (n + pb - 1) / pb;
     long long total = 0, longest = 0;
@@ -883,13 +886,13 @@ static int prefill_splits(int n, int hist, int nk, int window, int pb, int n_kv,
     const double step_us = 2.2, wg_us = 12.0, merge_bytes_per_us = 5.0e6;
     int best = 1;
     double best_us = 0.0;
-    for (int S = 1; S <= 4; S *= 2) {
+    for (int S = 1; S <= 16; S *= 2) {
         if (S > 1 && longest < 4LL * S) break;
         const double wgs = (double)nb * n_kv * S;
         const double floor_us = step_us * (double)((longest + S - 1) / S) + wg_us;
         const double spread_us = (step_us * (double)total + wg_us * wgs) / (double)(n_cu > 0 ? n_cu : 256);
         double t = floor_us > spread_us ? floor_us : spread_us;
-        if (S > 1) t += 3.0 + (double)(S + 1) * n * n_q * 256 * 4 / merge_bytes_per_us;
+        if (S > 1) t += (S > 4 ? 7.0 : 3.0) + (double)(S + 1) * n * n_q * 256 * 4 / merge_bytes_per_us;
         if (S == 1 || t < best_us) {
             best = S;
             best_us = t;
@@ -899,22 +902,24 @@ static int prefill_splits(int n, int hist, int nk, int window, int pb, int n_kv,
 }
 
 /* x8: the score policy, 1 = fp16 hi + fp8 cross terms, 0 = three fp16
- * passes (see prefill.hip). */
+ * passes (see prefill.hip).  The output goes to attn_out, or, when out_hi /
+ * out_lo are set, to those bf16 planes. */
 static int prefill_attention(g3attn_ctx *c, int layer, int start_pos, int n, const float *Q, const float *K,
                              const float *V, const uint16_t *q_norm, const uint16_t *k_norm, float *attn_out,
-                             int x8);
+                             uint16_t *out_hi, uint16_t *out_lo, int x8);
 
 int g3attn_prefill_device(g3attn_ctx *c, int layer, int start_pos, int n, const float *Q,
                           const float *K, const float *V, const uint16_t *q_norm,
                           const uint16_t *k_norm, float *attn_out) {
-    return prefill_attention(c, layer, start_pos, n, Q, K, V, q_norm, k_norm, attn_out, c ? c->prefill_x8 : 0);
+    return prefill_attention(c, layer, start_pos, n, Q, K, V, q_norm, k_norm, attn_out, NULL, NULL,
+                             c ? c->prefill_x8 : 0);
 }
 
 static int prefill_attention(g3attn_ctx *c, int layer, int start_pos, int n, const float *Q, const float *K,
                              const float *V, const uint16_t *q_norm, const uint16_t *k_norm, float *attn_out,
-                             int x8) {
+                             uint16_t *out_hi, uint16_t *out_lo, int x8) {
     if (!check_layer(c, layer, "g3attn_prefill") || !check_rope(c, "g3attn_prefill")) return G3_ERR_INVALID_ARG;
-    if (n < 0 || start_pos < 0 || (n > 0 && (!Q || !K || !V || !attn_out))) {
+    if (n < 0 || start_pos < 0 || (n > 0 && (!Q || !K || !V || (!attn_out && !out_hi)))) {
         set_err("g3attn_prefill: null buffer or negative start_pos / n");
         return G3_ERR_INVALID_ARG;
     }
@@ -1050,6 +1055,8 @@ static int prefill_attention(g3attn_ctx *c, int layer, int start_pos, int n, con
     pa.v_lo_flag = c->d_vflag;
     pa.epoch = c->pf_epoch;
     pa.out = attn_out;
+    pa.out_hi = out_hi;
+    pa.out_lo = out_lo;
     pa.ldk = ldk;
     pa.n = n;
     pa.hist = hist;
@@ -1511,7 +1518,7 @@ static size_t pb_products(const g3attn_ctx *c, int n) {
 }
 
 typedef struct {
-    float *x, *q, *k, *v, *attn, *t, *xn;
+    float *x, *q, *k, *v, *t, *xn;
     uint16_t *xh, *xl, *ah, *al, *hh, *hl;
 } pb_bufs;
 
@@ -1522,17 +1529,17 @@ static int pb_layout(g3attn_ctx *c, int n, int tail, pb_bufs *b) {
     const size_t hid = cfg->hidden_size, inter = cfg->intermediate_size;
     const size_t qs = (size_t)cfg->num_heads * D, ks = (size_t)cfg->num_kv_heads * D, N = n;
     const size_t t_n = pb_products(c, n), t_tail = pb_products(c, tail);
-    const size_t sz[13] = {N * hid * 4, N * qs * 4, N * ks * 4, N * ks * 4, N * qs * 4, (t_n > t_tail ? t_n : t_tail) * 4, hid * 4,
+    const size_t sz[12] = {N * hid * 4, N * qs * 4, N * ks * 4, N * ks * 4, (t_n > t_tail ? t_n : t_tail) * 4, hid * 4,
                            N * hid * 2, N * hid * 2, N * qs * 2, N * qs * 2, N * inter * 2, N * inter * 2};
     size_t total = 0;
-    for (int i = 0; i < 13; i++) total += align256(sz[i]);
+    for (int i = 0; i < 12; i++) total += align256(sz[i]);
     int rc = grow_buf(c, (float **)&c->d_pb, &c->d_pb_cap, total, "prefill activations");
     if (rc) return rc;
     unsigned char *p = (unsigned char *)c->d_pb;
-    void **dst[13] = {(void **)&b->x, (void **)&b->q, (void **)&b->k, (void **)&b->v, (void **)&b->attn,
-                      (void **)&b->t, (void **)&b->xn, (void **)&b->xh, (void **)&b->xl, (void **)&b->ah,
+    void **dst[12] = {(void **)&b->x, (void **)&b->q, (void **)&b->k, (void **)&b->v, (void **)&b->t,
+                      (void **)&b->xn, (void **)&b->xh, (void **)&b->xl, (void **)&b->ah,
                       (void **)&b->al, (void **)&b->hh, (void **)&b->hl};
-    for (int i = 0; i < 13; i++) {
+    for (int i = 0; i < 12; i++) {
         *dst[i] = p;
         p += align256(sz[i]);
     }
@@ -1603,19 +1610,9 @@ static int prefill_chunk(g3attn_ctx *c, const g3attn_weights *w, int n, int pos0
         /* the whole-model path keeps the exact score policy: its logits are
          * held to the token forward's 1e-4 x RMS, tighter than the
          * attention path's 2e-3 */
-        if ((rc = prefill_attention(c, l, pos0, n, b->q, b->k, b->v, lw->q_norm, lw->k_norm, b->attn, 0)))
+        if ((rc = prefill_attention(c, l, pos0, n, b->q, b->k, b->v, lw->q_norm, lw->k_norm, NULL, b->ah, b->al, 0)))
             return rc;
-        /* o_proj (:694-699) */
-        memset(&r, 0, sizeof r);
-        r.op = G3K_ROWS_SPLIT;
-        r.rows = n;
-        r.n = qs;
-        r.t = b->attn;
-        r.ldt = qs;
-        r.y_hi = b->ah;
-        r.y_lo = b->al;
-        r.ldy = qs;
-        if ((rc = rows_step(c, &r))) return rc;
+        /* o_proj (:694-699), on the planes the attention wrote */
         memset(&g, 0, sizeof g);
         g.x_hi = b->ah;
         g.x_lo = b->al;

@@ -296,6 +296,12 @@ inline float __shfl_xor(float v, int mask, int width = 64) {
     return __uint_as_float(r);
 }
 
+inline float __shfl(float v, int src) {
+    uint32_t r, unused;
+    hostemu::exchange(__float_as_uint(v), 0, src, &r, &unused);
+    return __uint_as_float(r);
+}
+
 inline float hostemu_exp2f(float x) { return exp2f(x); }
 #define __builtin_amdgcn_exp2f hostemu_exp2f
 
