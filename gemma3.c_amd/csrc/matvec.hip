@@ -200,9 +200,10 @@ __device__ __forceinline__ void pre_finish(const g3k_matvec_args &a, PreVals &v,
 // rows (a workgroup covers 4 RPW rows); with KS the workgroup's 4 waves share
 // RPW rows and wave w takes the w-th quarter of every row's chunks (one
 // memory round trip for long rows), the four partial sums meeting in LDS.
-template <int RPW, int CH, bool VEC, bool KS, bool GEGLU, bool PRE>
+template <int RPW, int CH, bool VEC, bool KS, bool GEGLU, bool PRE = false>
 __global__ __launch_bounds__(NT) void matvec_kernel(g3k_matvec_args a) {
     constexpr int NA = GEGLU ? 2 * RPW : RPW;
+    static_assert(!(VEC && PRE), "the vector path with a prologue is matvec_flow_kernel");
     __shared__ float red[KS ? NW : 1][NA];
     __shared__ float4 xs4[PRE ? G3K_MATVEC_PRE_MAX / 4 : 1];   // x formed by the residual prologue
     __shared__ float pre_red[NW];
@@ -238,8 +239,8 @@ __global__ __launch_bounds__(NT) void matvec_kernel(g3k_matvec_args a) {
             rs[t] = mat_rsrc(a.A[GEGLU ? t : m], (unsigned)((size_t)M * K * 2));
         uint4 w[NA][CH];
         float4 xa[CH], xb[CH];
-        // one round: CH chunks per lane of every row (and, without the
-        // prologue, the x chunks they meet) requested before any FMA
+        // one round: CH chunks per lane of every row and the x chunks they
+        // meet, requested before any FMA
         auto issue = [&](int base) {
 #pragma unroll
             for (int u = 0; u < CH; u++) {
@@ -251,31 +252,12 @@ __global__ __launch_bounds__(NT) void matvec_kernel(g3k_matvec_args a) {
                         uint4, __builtin_amdgcn_raw_buffer_load_b128(rs[GEGLU ? j / RPW : 0], roff[j] + 16u * (ok ? c : 0), 0, 2));
                     w[j][u] = ok ? t : make_uint4(0, 0, 0, 0);
                 }
-                if (!PRE) {
-                    xa[u] = ok ? x4[2 * c] : make_float4(0.f, 0.f, 0.f, 0.f);
-                    xb[u] = ok ? x4[2 * c + 1] : make_float4(0.f, 0.f, 0.f, 0.f);
-                }
+                xa[u] = ok ? x4[2 * c] : make_float4(0.f, 0.f, 0.f, 0.f);
+                xb[u] = ok ? x4[2 * c + 1] : make_float4(0.f, 0.f, 0.f, 0.f);
             }
         };
-        if (PRE) {
-            // the prologue's loads, then the first round's weights, which stay
-            // in flight while x is formed
-            PreVals pv;
-            pre_load(a, pv);
-            issue(cbeg);
-            pre_finish(a, pv, xs4, pre_red);
-        }
         for (int base = cbeg; base < cend; base += 64 * CH) {
-            if (!PRE || base != cbeg) issue(base);
-            if (PRE) {
-#pragma unroll
-                for (int u = 0; u < CH; u++) {
-                    const int c = base + lane + 64 * u;
-                    const bool ok = c < cend;
-                    xa[u] = ok ? xs4[2 * c] : make_float4(0.f, 0.f, 0.f, 0.f);
-                    xb[u] = ok ? xs4[2 * c + 1] : make_float4(0.f, 0.f, 0.f, 0.f);
-                }
-            }
+            issue(base);
 #pragma unroll
             for (int u = 0; u < CH; u++)
 #pragma unroll
@@ -320,16 +302,143 @@ __global__ __launch_bounds__(NT) void matvec_kernel(g3k_matvec_args a) {
     }
 }
 
+// The vector path with the residual prologue (K <= G3K_MATVEC_PRE_MAX): a
+// resident grid, two workgroups per CU, each forming x once and then
+// streaming rows.  Wave w of W takes items w, w + W, .. (an item: one row of
+// the Q / K / V matrices, or a gate row and its up row); its lanes hold their
+// NCH chunks of x in registers (chunk lane + 64 u of every row), and the loads
+// of the next two items are in flight while one is summed.  The first two
+// items' weights go out with the prologue's own loads, so the two norms hide
+// behind them.  One prologue per resident workgroup (15 MB of L2 reads in
+// all) instead of one per 4 rows is what lets the gate / up launch carry the
+// residual step too: at hidden 2560 the step's own launch took 4.3 us, and
+// folded into 5120 one-shot workgroups it cost more than that.
+constexpr int FLOW_WGS = 512;
+
+template <bool GEGLU, int NCH>
+__global__ __launch_bounds__(NT, 2) void matvec_flow_kernel(g3k_matvec_args a) {
+    constexpr int NA = GEGLU ? 2 : 1;
+    constexpr int NB = GEGLU && NCH > 6 ? 2 : 3;   // items in registers (256 VGPRs at two waves per SIMD)
+    __shared__ float4 xs4[G3K_MATVEC_PRE_MAX / 4];
+    __shared__ float pre_red[NW];
+    const int K = a.K, nch = K >> 3;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int items = a.M[0];
+    for (int m = 1; m < a.n_mat && !GEGLU; m++) items += a.M[m];
+    const int waves = gridDim.x * NW, first = blockIdx.x * NW + wave;
+    // item -> matrix (GEGLU: 0) and row
+    auto locate = [&](int it, int &m, int &row) {
+        row = it;
+        m = 0;
+        while (!GEGLU && row >= a.M[m]) row -= a.M[m++];
+    };
+    uint4 w[NB][NA][NCH];
+    auto issue = [&](int b, int it) {
+        int m, row;
+        locate(it, m, row);
+        const unsigned base = (unsigned)row * (unsigned)K * 2u;
+#pragma unroll
+        for (int j = 0; j < NA; j++) {
+            const __amdgpu_buffer_rsrc_t rs = mat_rsrc(a.A[GEGLU ? j : m], (unsigned)((size_t)a.M[m] * K * 2));
+#pragma unroll
+            for (int u = 0; u < NCH; u++) {
+                const int c = lane + 64 * u;   // only the last chunk of a row can end inside the wave
+                w[b][j][u] = __builtin_bit_cast(
+                    uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, 16u * (u + 1 < NCH || c < nch ? c : 0), base, 2));
+            }
+        }
+    };
+    PreVals pv;
+    pre_load(a, pv);
+    // past the end (a grid with more waves than items) the last item
+#pragma unroll
+    for (int b = 0; b + 1 < NB; b++) issue(b, min(first + b * waves, items - 1));
+    pre_finish(a, pv, xs4, pre_red);
+    const bool tail = lane + 64 * (NCH - 1) < nch;
+    float4 xa[NCH], xb[NCH];
+#pragma unroll
+    for (int u = 0; u < NCH; u++) {
+        const bool ok = u + 1 < NCH || tail;
+        const int c = ok ? lane + 64 * u : 0;
+        xa[u] = ok ? xs4[2 * c] : make_float4(0.f, 0.f, 0.f, 0.f);
+        xb[u] = ok ? xs4[2 * c + 1] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    auto sum = [&](int b, int it) {
+        float tot[NA];
+#pragma unroll
+        for (int j = 0; j < NA; j++) {
+            if (!tail) w[b][j][NCH - 1] = make_uint4(0, 0, 0, 0);
+            float acc = 0.f;
+#pragma unroll
+            for (int u = 0; u < NCH; u++) acc += dot8(w[b][j][u], xa[u], xb[u]);
+            tot[j] = wave_sum(acc);
+        }
+        if (lane == 0) {
+            int m, row;
+            locate(it, m, row);
+            a.y[m][row] = GEGLU ? gelu_tanh(tot[0]) * tot[NA - 1] : tot[0];
+        }
+    };
+    // Whole rounds of NB items, each with the request NB - 1 items ahead;
+    // then what is left, without (a branch around a request would make the
+    // compiler wait for it at the join).
+    int it = first;
+    for (; it + (2 * NB - 2) * waves < items; it += NB * waves) {
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            issue((b + NB - 1) % NB, it + (b + NB - 1) * waves);
+            sum(b, it + b * waves);
+        }
+    }
+    const int left = it < items ? (items - it + waves - 1) / waves : 0;   // uniform, at most 2 NB - 2
+#pragma unroll
+    for (int n = 1; n <= 2 * NB - 2; n++) {
+        if (left != n) continue;
+#pragma unroll
+        for (int i = 0; i < n; i++) {
+            if (i + NB - 1 < n) issue((i + NB - 1) % NB, it + (i + NB - 1) * waves);
+            sum(i % NB, it + i * waves);
+        }
+    }
+}
+
+template <bool GEGLU, int NCH>
+hipError_t launch_flow_n(const g3k_matvec_args *a, hipStream_t st) {
+    long long items = a->M[0];
+    for (int m = 1; m < a->n_mat && !GEGLU; m++) items += a->M[m];
+    const long long wgs = (items + NW - 1) / NW;
+    hipLaunchKernelGGL((matvec_flow_kernel<GEGLU, NCH>), dim3((unsigned)(wgs < FLOW_WGS ? wgs : FLOW_WGS)), dim3(NT), 0,
+                       st, *a);
+    return hipGetLastError();
+}
+
+template <bool GEGLU>
+hipError_t launch_flow(const g3k_matvec_args *a, hipStream_t st) {
+    switch ((a->K / 8 + 63) / 64) {
+        case 1: return launch_flow_n<GEGLU, 1>(a, st);
+        case 2: return launch_flow_n<GEGLU, 2>(a, st);
+        case 3: return launch_flow_n<GEGLU, 3>(a, st);
+        case 4: return launch_flow_n<GEGLU, 4>(a, st);
+        case 5: return launch_flow_n<GEGLU, 5>(a, st);
+        case 6: return launch_flow_n<GEGLU, 6>(a, st);
+        case 7: return launch_flow_n<GEGLU, 7>(a, st);
+        default: return launch_flow_n<GEGLU, 8>(a, st);
+    }
+}
+
 template <int RPW, int CH, bool VEC, bool KS = false, bool GEGLU = false>
 hipError_t launch(const g3k_matvec_args *a, hipStream_t st) {
     int blocks = 0;
     const int nm = GEGLU ? 1 : a->n_mat;
     const int rows_per_wg = KS ? RPW : NW * RPW;
     for (int m = 0; m < nm; m++) blocks += (a->M[m] + rows_per_wg - 1) / rows_per_wg;
-    if (a->pre_t)
-        hipLaunchKernelGGL((matvec_kernel<RPW, CH, VEC, KS, GEGLU, true>), dim3(blocks), dim3(NT), 0, st, *a);
-    else
-        hipLaunchKernelGGL((matvec_kernel<RPW, CH, VEC, KS, GEGLU, false>), dim3(blocks), dim3(NT), 0, st, *a);
+    if constexpr (!VEC) {
+        if (a->pre_t) {
+            hipLaunchKernelGGL((matvec_kernel<RPW, CH, VEC, KS, GEGLU, true>), dim3(blocks), dim3(NT), 0, st, *a);
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((matvec_kernel<RPW, CH, VEC, KS, GEGLU>), dim3(blocks), dim3(NT), 0, st, *a);
     return hipGetLastError();
 }
 
@@ -361,9 +470,11 @@ extern "C" int g3k_matvec(const g3k_matvec_args *a, void *stream) {
     hipStream_t st = (hipStream_t)stream;
     if (a->mode == G3K_MV_GEGLU) {
         if (a->n_mat != 2 || a->M[0] != a->M[1]) return (int)hipErrorInvalidValue;
+        if (vec && pre) return (int)launch_flow<true>(a, st);
         return (int)(vec ? launch<2, 2, true, true, true>(a, st) : launch<2, 1, false, true, true>(a, st));
     }
     if (a->mode != 0) return (int)hipErrorInvalidValue;
+    if (vec && pre) return (int)launch_flow<false>(a, st);
     if (!vec) return (int)(rows >= 16384 ? launch<2, 1, false>(a, st) : launch<1, 1, false>(a, st));
     // two rows per wave once there are enough rows to fill the chip with them
     if (rows >= 16384) return (int)launch<2, 8, true>(a, st);

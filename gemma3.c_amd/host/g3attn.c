@@ -373,7 +373,7 @@ g3attn_ctx *g3attn_create(const g3attn_config *cfg, int max_context,
         const char *nt = getenv("G3ATTN_DECODE_NT");
         c->nt_loads = nt ? atoi(nt) : 2;
         const char *ff = getenv("G3ATTN_FORWARD_FOLD");
-        c->forward_fold = ff ? atoi(ff) & 3 : 1;
+        c->forward_fold = ff ? atoi(ff) & 3 : 3;
         if (c->min_rows < G3K_SPLIT_GRAIN) c->min_rows = G3K_SPLIT_GRAIN;
     }
 
