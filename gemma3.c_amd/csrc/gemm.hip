@@ -12,9 +12,9 @@
 // with fp32 accumulation: twice the algorithmic MFMA work, within a few
 // 2^-17 of the reference's fp32 sgemm.
 //
-// Tiling.  Three forms of gemm_kernel, picked by g3k_gemm_plan: Pairs (many
-// tokens), Stream in two widths (few tokens) and Gate (GEGLU over the most
-// tokens); each says what bounds it.  In all of them W and x tiles move
+// Tiling.  Two forms of gemm_kernel, picked by g3k_gemm_plan: Pairs (many
+// tokens) and Stream in two widths (few tokens); each says what bounds it.  In
+// both W and x tiles move
 // from global memory straight into LDS with buffer -> LDS loads
 // (buffer_load_dwordx4 ... lds, one wave instruction = 1 KiB).  Rows beyond M
 // or N read zero (the buffer descriptor's range check), so ragged tiles need
@@ -38,7 +38,6 @@ namespace {
 using namespace g3k;
 
 constexpr int BN = 128, BK = 32, NT = 256;
-constexpr int TILE_B = 128 * BK * 2;   // one operand tile in LDS: 8 KiB
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -46,32 +45,6 @@ typedef __attribute__((address_space(3))) void *lds_ptr;
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)bytes, 0x00020000);
-}
-
-// Byte offset, inside a tile, of chunk c (8 k values) of row r.
-__device__ __forceinline__ int tile_off(int r, int c) {
-    return ((r >> 4) * 64 + (r & 15) * 4 + (c ^ ((r >> 2) & 3))) * 16;
-}
-
-// Copy rows row0 .. row0 + 127, k0 .. k0 + 31 of a [rows][ld] bf16 matrix
-// into an LDS tile.  Wave w moves the 16-row groups w and w + 4; lane i of
-// a group instruction lands at byte 16 i of the group, which is slot i =
-// 4 r + c' with c' = c ^ (r / 4 % 4).
-__device__ __forceinline__ void fetch_tile(__amdgpu_buffer_rsrc_t rs, char *tile, int row0, int ld, int k0,
-                                           int wave, int lane) {
-    const int r = lane >> 2, cp = lane & 3;
-    const int c = cp ^ ((r >> 2) & 3);
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int g = wave + 4 * h;
-        const int row = row0 + g * 16 + r;
-        const uint32_t voff = (uint32_t)row * (uint32_t)ld * 2u + (uint32_t)(k0 + c * 8) * 2u;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr)(tile + g * 1024), 16, voff, 0, 0, 0);
-    }
-}
-
-__device__ __forceinline__ bf16x8 frag(const char *tile, int r, int c) {
-    return *reinterpret_cast<const bf16x8 *>(tile + tile_off(r, c));
 }
 
 __device__ __forceinline__ float gelu_tanh(float x) {
@@ -123,84 +96,6 @@ __device__ __forceinline__ float *out_base(const g3k_gemm_args &a, int m, int z,
     return a.part + (size_t)z * a.N * ld + col;
 }
 
-// GEGLU over many tokens: 128 gate rows and the same 128 up rows x 128 tokens
-// per workgroup of 4 waves, two workgroups per CU (64 KiB of LDS each, two
-// stages of 32 k values).  Wave (wm, wn) owns 64 gate rows, the same 64 up
-// rows and tokens wn * 64 .. + 63; per k step it reads 8 W fragments and 8 x
-// fragments (4 hi, 4 lo) for 64 MFMAs.
-struct Gate {
-    static constexpr int THREADS = NT, WAVES = 2;
-    static __device__ void run(const g3k_gemm_args &a);
-};
-__device__ __forceinline__ void Gate::run(const g3k_gemm_args &a) {
-    constexpr int MT = 8;
-    constexpr int W_B = 2 * TILE_B;
-    constexpr int STAGE_B = W_B + 2 * TILE_B;
-    __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE_B];
-
-    const int M = a.M[0], K = a.K, N = a.N;
-    const int m0 = blockIdx.x * 128, n0 = blockIdx.y * BN;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave & 1, wn = wave >> 1;
-
-    const uint32_t wbytes = (uint32_t)((size_t)M * K * 2);
-    const __amdgpu_buffer_rsrc_t rw0 = rsrc(a.W[0], wbytes), rw1 = rsrc(a.W[1], wbytes);
-    const uint32_t xbytes = (uint32_t)((size_t)N * a.ldx * 2);
-    const __amdgpu_buffer_rsrc_t rxh = rsrc(a.x_hi, xbytes), rxl = rsrc(a.x_lo, xbytes);
-
-    f32x4 acc[MT][4];
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-        for (int nt = 0; nt < 4; nt++) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    auto fetch = [&](int s, int k0) {
-        char *st = smem + s * STAGE_B;
-        fetch_tile(rw0, st, m0, K, k0, wave, lane);
-        fetch_tile(rw1, st + TILE_B, m0, K, k0, wave, lane);
-        fetch_tile(rxh, st + W_B, n0, a.ldx, k0, wave, lane);
-        fetch_tile(rxl, st + W_B + TILE_B, n0, a.ldx, k0, wave, lane);
-    };
-
-    const int nk = K / BK;
-    const int fr = lane & 15, fc = lane >> 4;
-    fetch(0, 0);
-    for (int kt = 0; kt < nk; kt++) {
-        __syncthreads();   // stage kt has landed; stage kt + 1's slot is free
-        if (kt + 1 < nk) fetch((kt + 1) & 1, (kt + 1) * BK);
-        const char *st = smem + (kt & 1) * STAGE_B;
-        bf16x8 bh[4], bl[4];
-#pragma unroll
-        for (int nt = 0; nt < 4; nt++) {
-            bh[nt] = frag(st + W_B, wn * 64 + nt * 16 + fr, fc);
-            bl[nt] = frag(st + W_B + TILE_B, wn * 64 + nt * 16 + fr, fc);
-        }
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            // W region row of the wave's tile mt: gate tiles 0..3, up tiles 4..7
-            const bf16x8 w = frag(st, (mt >> 2) * 128 + wm * 64 + (mt & 3) * 16 + fr, fc);
-#pragma unroll
-            for (int nt = 0; nt < 4; nt++) {
-                acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, bh[nt], acc[mt][nt], 0, 0, 0);
-                acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, bl[nt], acc[mt][nt], 0, 0, 0);
-            }
-        }
-    }
-
-    // epilogue: lane holds rows m = base + 4 (l / 16) + i, i = 0..3, of token l % 16
-#pragma unroll
-    for (int mt = 0; mt < MT / 2; mt++)
-#pragma unroll
-        for (int nt = 0; nt < 4; nt++) {
-            const int m = m0 + wm * 64 + mt * 16 + 4 * fc, n = n0 + wn * 64 + nt * 16 + fr;
-            if (n >= N || m >= M) continue;   // M is a multiple of 4 (checked on the host)
-            const f32x4 g = acc[mt][nt], u = acc[mt + 4][nt];
-            store_planes(a, n, m, gelu_tanh(g[0]) * u[0], gelu_tanh(g[1]) * u[1], gelu_tanh(g[2]) * u[2],
-                         gelu_tanh(g[3]) * u[3]);
-        }
-}
-
 // ---------------------------------------------------------------------------
 // Many tokens: 256 weight rows (GEGLU: 128 gate rows and the same 128 up
 // rows) x 128 tokens per workgroup of 8 waves, one workgroup per CU, K in
@@ -215,8 +110,11 @@ __device__ __forceinline__ void Gate::run(const g3k_gemm_args &a) {
 // Against 128- and 256-row x 128-token tiles with 32-wide stages, two
 // workgroups per CU (us, Gemma3-4B shapes): 8192 tokens: Q/K/V 349 -> 338,
 // o_proj 185 -> 180, down_proj 896 -> 781; 2048: 88 -> 72, 56 -> 54, 300 ->
-// 193; 512: 53 -> 26, 22 -> 22, 79 -> 62, gate + up 136 -> 132; 256: gate +
-// up 95 -> 72.  The K loop is bound by the matrix cores at the clocks they
+// 193; 512: 53 -> 26, 22 -> 22, 79 -> 62; gate + up at 256 / 512 / 1024 / 2048
+// / 8192: 97 -> 72, 136 -> 128, 248 -> 205, 447 -> 382, 1509 -> 1422 (1.21
+// PFLOP/s issued, what a library bf16 product of that size reaches here).
+// A single 64-wide stage per workgroup and two of them per CU in turn measured
+// the same at 8192 and slower below (gate + up 407 at 2048).  The K loop is bound by the matrix cores at the clocks they
 // sustain and by the L2 -> LDS stream about equally (down_proj at 8192
 // without its fetches: 602 us; with a quarter of its MFMAs: 645).
 template <bool GEGLU>
@@ -473,7 +371,7 @@ __device__ __forceinline__ void Stream<MT, NTL, DEPTH, NWV, OCC>::run(const g3k_
         }
 }
 
-// One launch of form F (Stream, Pairs, Gate).
+// One launch of form F (Stream, Pairs).
 template <class F>
 __global__ __launch_bounds__(F::THREADS, F::WAVES) void gemm_kernel(g3k_gemm_args a) {
     F::run(a);
@@ -558,8 +456,6 @@ int launch_form(const g3k_gemm_args *a, hipStream_t st) {
             if (a->N <= 32) return launch_stream<Stream<1, 2, 3, 4, 2>>(a, st);
             if (narrow_tokens(a->N) == 48) return launch_stream<Stream<1, 3, 3, 4, 2>>(a, st);
             return launch_stream<Stream<1, 4, 2, 4, 3>>(a, st);
-        case G3K_GEMM_GATE:
-            return launch<Gate>(a, (a->M[0] + 127) / 128, nb, st);
         default:
             if (a->mode == G3K_MV_GEGLU) return launch<Pairs<true>>(a, (a->M[0] + 127) / 128, nb, st);
             return launch<Pairs<false>>(a, row_tiles(a, 256), nb, st);
@@ -578,8 +474,7 @@ int launch_form(const g3k_gemm_args *a, hipStream_t st) {
 //   of n_cu workgroups (1.75 us per 64-wide chunk and 5 us around the K loop,
 //   measured with every CU busy) and its partial products (moved at about 8
 //   MB per us); the S with the least total is taken.
-// - GEGLU from 1536 tokens on fills several rounds of any tile, and two small
-//   workgroups per CU hide each other's epilogues: 408 us against 434 at 2048.
+// - GEGLU takes the tiles unsplit.
 extern "C" void g3k_gemm_plan(int N, int K, int n_mat, const int *M, int geglu, int consumer_adds, int n_cu, int *kind,
                               int *ksplit) {
     long long sum = 0, tiles64 = 0, tiles256 = 0;
@@ -605,11 +500,8 @@ extern "C" void g3k_gemm_plan(int N, int K, int n_mat, const int *M, int geglu, 
         return;
     }
     *ksplit = 1;
-    if (geglu) {
-        *kind = N >= 1536 ? G3K_GEMM_GATE : G3K_GEMM_TILE;
-        return;
-    }
     *kind = G3K_GEMM_TILE;
+    if (geglu) return;
     const long long tiles = tiles256 * ((N + BN - 1) / BN);
     double best = 0.0;
     for (int s = 1; s <= 16 && s <= most; s++) {
@@ -630,8 +522,7 @@ extern "C" int g3k_gemm(const g3k_gemm_args *a, void *stream) {
         return (int)hipErrorInvalidValue;
     if (a->n_mat < 1 || a->n_mat > G3K_MATVEC_MAX || (geglu && a->n_mat != 2) || (a->mode != 0 && !geglu))
         return (int)hipErrorInvalidValue;
-    if (a->kind < G3K_GEMM_TILE || a->kind > G3K_GEMM_GATE || (a->kind == G3K_GEMM_GATE && !geglu))
-        return (int)hipErrorInvalidValue;
+    if (a->kind < G3K_GEMM_TILE || a->kind > G3K_GEMM_NARROW) return (int)hipErrorInvalidValue;
     // at least one 64-wide chunk per split; the grid's y and z limits
     const bool stream_w = a->kind == G3K_GEMM_WIDE || a->kind == G3K_GEMM_NARROW;
     if (S < 1 || S > (a->K + 63) / 64 || S > 65535 || a->N > (stream_w ? 16 : BN) * 65535)

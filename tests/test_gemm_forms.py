@@ -21,7 +21,7 @@ from helpers import DeviceBuffer, g3attn
 from test_attn_hostemu import Emu, built  # noqa: F401  (built: the emulator's build)
 
 G = g3attn()
-TILE, WIDE, NARROW, GATE = range(4)
+TILE, WIDE, NARROW = range(3)
 
 
 def plan(N, K, M, geglu=0, consumer_adds=0, n_cu=256):
@@ -46,7 +46,7 @@ def test_plan_stays_in_the_launchers_limits(K):
                     assert 4 * s * N * sum(M) <= 256e6, (N, M, s)
         kind, s = plan(N, K, [10240, 10240], 1)
         assert 1 <= s <= (K + 63) // 64
-        assert kind == (WIDE if N <= 128 else TILE if N < 1536 else GATE)
+        assert kind == (WIDE if N <= 128 else TILE)
         assert s == 1 or kind == WIDE
 
 
