@@ -151,6 +151,10 @@ int g3k_rope_write(const g3k_rope_write_args *a, void *stream);
 int g3k_kv_scatter(float *dst_k, float *dst_v, float *rows_k, float *rows_v, int n, int n_kv_heads,
                    long long head_stride, int slot, int to_rows, void *stream);
 
+/* A small host -> device copy by a kernel: src is the device address of pinned
+ * host memory, both 16-byte aligned, bytes a multiple of 16. */
+int g3k_host_copy(void *dst, const void *src, int bytes, void *stream);
+
 /* Prefill staging of key rows kk0..kk0+cnt-1 (key index kk = position -
  * kstart): K (already normed + rotated, fp32) -> key rows of
  * kq [H_kv][ldk][2][D] in the format kscale selects (exact fp16 hi | lo, or

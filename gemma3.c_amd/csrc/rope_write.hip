@@ -77,3 +77,23 @@ extern "C" int g3k_kv_scatter(float *dst_k, float *dst_v, float *rows_k, float *
                        rows_k, rows_v, n, n_kv_heads, head_stride, slot, to_rows);
     return (int)hipGetLastError();
 }
+
+namespace {
+
+// 16 bytes per thread: a few KiB of pinned host memory -> device, one PCIe
+// round trip for all of it.
+__global__ __launch_bounds__(256) void host_copy_kernel(uint4 *dst, const uint4 *src, int words) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < words) dst[i] = src[i];
+}
+
+}  // namespace
+
+extern "C" int g3k_host_copy(void *dst, const void *src, int bytes, void *stream) {
+    if (bytes <= 0) return 0;
+    if (bytes % 16 || (((uintptr_t)dst | (uintptr_t)src) & 15)) return (int)hipErrorInvalidValue;
+    const int words = bytes / 16;
+    hipLaunchKernelGGL(host_copy_kernel, dim3((words + 255) / 256), dim3(256), 0, (hipStream_t)stream, (uint4 *)dst,
+                       (const uint4 *)src, words);
+    return (int)hipGetLastError();
+}

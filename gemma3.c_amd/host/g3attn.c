@@ -100,9 +100,12 @@ struct g3attn_ctx {
     float **kc, **vc;
     int *rows;
     float *ws_acc, *ws_ml;
-    /* staging of the host-pointer decode: q | k | v | q_norm | k_norm, and out */
+    /* staging of the host-pointer decode: q | k | v | q_norm | k_norm, and
+     * out.  The GPU reads h_in and writes h_out (pinned) through their device
+     * addresses; d_in is the inputs' device copy. */
     unsigned char *h_in, *d_in;
-    float *h_out, *d_out;
+    float *h_out;
+    void *h_in_dev, *h_out_dev;
     size_t in_bytes;
     /* grow-on-demand device buffers for host-pointer batch calls */
     void *d_big;
@@ -196,7 +199,6 @@ static void ctx_free(g3attn_ctx *c) {
     hipFree(c->ws_acc);
     hipFree(c->ws_ml);
     hipFree(c->d_in);
-    hipFree(c->d_out);
     hipFree(c->d_big);
     hipFree(c->d_pf);
     hipFree(c->d_vflag);
@@ -382,7 +384,9 @@ g3attn_ctx *g3attn_create(const g3attn_config *cfg, int max_context,
     if (hipHostMalloc((void **)&c->h_in, c->in_bytes, 0) != hipSuccess) goto fail_rt;
     if (hipHostMalloc((void **)&c->h_out, qs * sizeof(float), 0) != hipSuccess) goto fail_rt;
     if (!alloc_dev((void **)&c->d_in, c->in_bytes, "staging")) goto fail;
-    if (!alloc_dev((void **)&c->d_out, qs * sizeof(float), "staging")) goto fail;
+    if (hipHostGetDevicePointer(&c->h_in_dev, c->h_in, 0) != hipSuccess ||
+        hipHostGetDevicePointer(&c->h_out_dev, c->h_out, 0) != hipSuccess)
+        goto fail_rt;
     if (hipDeviceSynchronize() != hipSuccess) goto fail_rt;
     return c;
 
@@ -711,15 +715,18 @@ int g3attn_decode(g3attn_ctx *c, int layer, int pos, const float *q, const float
         memcpy(h + nb, q_norm, D * sizeof(uint16_t));
         memcpy(h + nb + D * 2, k_norm, D * sizeof(uint16_t));
     }
-    HIP_TRY(hipMemcpyAsync(c->d_in, h, norm ? c->in_bytes : nb, hipMemcpyHostToDevice, c->stream),
-            "g3attn_decode upload");
+    /* The inputs are a few tens of KiB and the output is written once: a
+     * kernel that reads them over PCIe and a decode that writes its output
+     * there take two copy commands (and their queue hand-overs) out of the
+     * call.  The decode's own workgroups read q many times, so they read the
+     * device copy.  2000 positions, 16 / 8 heads: 42.0 -> 37.3 us a call. */
+    int rc = g3k_host_copy(c->d_in, c->h_in_dev, (int)(norm ? c->in_bytes : nb), c->stream);
+    if (rc) return hip_fail((hipError_t)rc, "g3attn_decode upload");
     const float *dq = (const float *)c->d_in;
-    int rc = g3attn_decode_device(c, layer, pos, dq, dq + qs, dq + qs + ks,
-                                  norm ? (const uint16_t *)(c->d_in + nb) : NULL,
-                                  norm ? (const uint16_t *)(c->d_in + nb + D * 2) : NULL, c->d_out);
+    rc = g3attn_decode_device(c, layer, pos, dq, dq + qs, dq + qs + ks,
+                              norm ? (const uint16_t *)(c->d_in + nb) : NULL,
+                              norm ? (const uint16_t *)(c->d_in + nb + D * 2) : NULL, (float *)c->h_out_dev);
     if (rc) return rc;
-    HIP_TRY(hipMemcpyAsync(c->h_out, c->d_out, qs * sizeof(float), hipMemcpyDeviceToHost, c->stream),
-            "g3attn_decode download");
     HIP_TRY(hipStreamSynchronize(c->stream), "g3attn_decode");
     memcpy(attn_out, c->h_out, qs * sizeof(float));
     return G3_OK;

@@ -129,6 +129,10 @@ hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) {
     *p = aligned(bytes);
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }
+hipError_t hipHostGetDevicePointer(void **dev, void *host, unsigned) {
+    *dev = host;
+    return hipSuccess;
+}
 hipError_t hipHostFree(void *p) {
     g_alloc_calls++;
     std::free(p);
