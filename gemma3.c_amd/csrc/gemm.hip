@@ -253,27 +253,32 @@ __device__ __forceinline__ void Pairs<GEGLU>::run(const g3k_gemm_args &a) {
 // and all the tokens, and K is split until the grid fills the chip.  K moves
 // in chunks of 64: one DMA instruction takes 8 rows x 128 B (a whole line of
 // each row: 16 rows x 64 B, the MFMA operand's own shape, read W at 2.3-4.0
-// TB/s against 5.0-5.5), and DEPTH chunks are in flight in an LDS ring whose
-// barrier waits only for the oldest.  A row's eight 16-byte pieces sit at
+// TB/s against 5.0-5.5), and the next chunks are in flight in two LDS rings, DW
+// slots of W and DX of x, whose barrier waits only for the oldest.  Where two
+// chunks of 96 or 128 tokens fill the LDS, x (from the L2) keeps two slots and
+// W (from memory) takes the rest as a third: gate and up of 77 tokens, 2 x
+// 10240 x 2560: 32.4 -> 30.0 us.  (One workgroup of 128 rows x 96 or 128
+// tokens with these rings instead of 64 rows x 48 or 64, for the other
+// products: down_proj of 100 tokens 21.1 -> 26.0 us, twice the splits.)  A row's eight 16-byte pieces sit at
 // c ^ (row % 8), so a fragment read (16 rows, one piece) spreads over the
 // banks.  Rows past M or N read zero; rows of a last half chunk past K hold
 // other rows' values and are not multiplied.
 // Every split writes fp32 partial products; the consumer or
 // split_reduce_kernel adds them in split order.
-template <int MT, int NTL, int DEPTH, int NWV, int OCC>
+template <int MT, int NTL, int DW, int DX, int NWV, int OCC>
 struct Stream {
     static constexpr int THREADS = NWV * 64, WAVES = OCC, ROWS = NWV * MT * 16, TOKENS = NTL * 16;
     static __device__ void run(const g3k_gemm_args &a);
 };
-template <int MT, int NTL, int DEPTH, int NWV, int OCC>
-__device__ __forceinline__ void Stream<MT, NTL, DEPTH, NWV, OCC>::run(const g3k_gemm_args &a) {
+template <int MT, int NTL, int DW, int DX, int NWV, int OCC>
+__device__ __forceinline__ void Stream<MT, NTL, DW, DX, NWV, OCC>::run(const g3k_gemm_args &a) {
     constexpr int BM = NWV * MT * 16, KC = 64;
     constexpr int W_B = BM * KC * 2, X_B = NTL * 16 * KC * 2;   // X_B: one plane
-    constexpr int STAGE_B = W_B + 2 * X_B;
     constexpr int NWI = MT * 2;             // W fetches of a wave per chunk (8 rows each)
     constexpr int NXI = NTL * 4 / NWV;      // its x_hi / x_lo fetches
     static_assert(NTL * 4 % NWV == 0, "every wave issues the same number of fetches (counted waits)");
-    __shared__ __attribute__((aligned(1024))) char smem[DEPTH * STAGE_B];
+    static_assert(DX >= 2 && (DW == DX || DW == DX + 1), "a deeper W ring would drain at x's wait");
+    __shared__ __attribute__((aligned(1024))) char smem[DW * W_B + DX * 2 * X_B];
 
     int bx = blockIdx.x, m_idx = 0;
     while (m_idx + 1 < a.n_mat && bx >= (a.M[m_idx] + BM - 1) / BM) {
@@ -303,36 +308,43 @@ __device__ __forceinline__ void Stream<MT, NTL, DEPTH, NWV, OCC>::run(const g3k_
 #pragma unroll
         for (int nt = 0; nt < NTL; nt++) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // chunk c (clamped to the split's last: the counted waits want every
-    // round to issue the same number) into ring slot s
-    auto fetch = [&](int s, int c) {
+    // W and x of chunk c (clamped to the split's last: the counted waits want
+    // every round to issue the same number) into slot s of their rings
+    auto fetch_w = [&](int s, int c) {
         const uint32_t kb = (uint32_t)(c < c1 ? c : c1 - 1) * (KC * 2);
-        char *ws = smem + s * STAGE_B + wave * (MT * 2048);
+        char *ws = smem + s * W_B + wave * (MT * 2048);
 #pragma unroll
         for (int i = 0; i < NWI; i++) fetch8(rw, ws + i * 1024, wbase + (uint32_t)i * (uint32_t)K * 16u, kb);
-        char *xs = smem + s * STAGE_B + W_B;
+    };
+    auto fetch_x = [&](int s, int c) {
+        const uint32_t kb = (uint32_t)(c < c1 ? c : c1 - 1) * (KC * 2);
+        char *xs = smem + DW * W_B + s * (2 * X_B);
 #pragma unroll
         for (int j = 0; j < NXI; j++) {
             const int g = wave + NWV * j, r8 = g % (2 * NTL);   // 8-row group r8 of plane g / (2 NTL)
             fetch8(g < 2 * NTL ? rxh : rxl, xs + g * 1024, xbase + (uint32_t)r8 * (uint32_t)a.ldx * 16u, kb);
         }
     };
-    // The ring's waits count fetches in issue order, so no round may move
-    // into another: a scheduling fence after each.
+    // The rings' waits count fetches in issue order, so no round may move
+    // into another: a scheduling fence after each.  The round of chunk c
+    // fetches x of chunk c + DX - 1, then W of chunk c + DW - 1.
 #pragma unroll
-    for (int d = 0; d < DEPTH - 1; d++) {
-        fetch(d, c0 + d);
+    for (int d = 1 - DW; d < 0; d++) {
+        if (d + DX - 1 >= 0) fetch_x(d + DX - 1, c0 + d + DX - 1);
+        fetch_w(d + DW - 1, c0 + d + DW - 1);
         G3K_ORDER_FENCE();
     }
     const int f0 = fr * 128 + ((fc ^ (fr & 7)) * 16), f1 = fr * 128 + (((4 + fc) ^ (fr & 7)) * 16);
-    int slot = 0;
+    int sw = 0, sx = 0;
     for (int c = c0; c < c1; c++) {
-        // chunk c has landed (the DEPTH - 2 rounds after it may be in flight)
-        // and every wave is done with chunk c - 1, whose slot is filled next
-        G3K_WAIT_BARRIER((DEPTH - 2) * (NWI + NXI));
-        fetch(slot == 0 ? DEPTH - 1 : slot - 1, c + DEPTH - 1);
+        // chunk c has landed (the DX - 2 rounds after its x, and the W fetched
+        // after it, may be in flight) and every wave is done with chunk c - 1,
+        // whose slots are filled next
+        G3K_WAIT_BARRIER((DX - 2) * (NWI + NXI) + (DW > DX ? NWI : 0));
+        fetch_x(sx == 0 ? DX - 1 : sx - 1, c + DX - 1);
+        fetch_w(sw == 0 ? DW - 1 : sw - 1, c + DW - 1);
         G3K_ORDER_FENCE();
-        const char *ws = smem + slot * STAGE_B + wave * (MT * 2048), *xs = smem + slot * STAGE_B + W_B;
+        const char *ws = smem + sw * W_B + wave * (MT * 2048), *xs = smem + DW * W_B + sx * (2 * X_B);
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
             if (kk == 1 && c * KC + 32 >= K) break;   // uniform: K ends with half a chunk
@@ -352,7 +364,8 @@ __device__ __forceinline__ void Stream<MT, NTL, DEPTH, NWV, OCC>::run(const g3k_
                     acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[mt], xl, acc[mt][nt], 0, 0, 0);
             }
         }
-        slot = slot + 1 == DEPTH ? 0 : slot + 1;
+        sw = sw + 1 == DW ? 0 : sw + 1;
+        sx = sx + 1 == DX ? 0 : sx + 1;
     }
     // the clamped fetches past the end still write the ring
     G3K_WAIT_VMEM();
@@ -447,15 +460,15 @@ int launch_form(const g3k_gemm_args *a, hipStream_t st) {
     const int nb = (a->N + BN - 1) / BN;
     switch (a->kind) {
         case G3K_GEMM_WIDE:
-            if (a->N <= 32) return launch_stream<Stream<2, 2, 3, 8, 1>>(a, st);
-            if (a->N <= 64) return launch_stream<Stream<2, 4, 3, 8, 1>>(a, st);
-            if (a->N <= 96) return launch_stream<Stream<2, 6, 2, 8, 1>>(a, st);
-            return launch_stream<Stream<2, 8, 2, 8, 1>>(a, st);
+            if (a->N <= 32) return launch_stream<Stream<2, 2, 3, 3, 8, 1>>(a, st);
+            if (a->N <= 64) return launch_stream<Stream<2, 4, 3, 3, 8, 1>>(a, st);
+            if (a->N <= 96) return launch_stream<Stream<2, 6, 3, 2, 8, 1>>(a, st);
+            return launch_stream<Stream<2, 8, 3, 2, 8, 1>>(a, st);
         case G3K_GEMM_NARROW:
-            if (a->N <= 16) return launch_stream<Stream<1, 1, 5, 4, 2>>(a, st);
-            if (a->N <= 32) return launch_stream<Stream<1, 2, 3, 4, 2>>(a, st);
-            if (narrow_tokens(a->N) == 48) return launch_stream<Stream<1, 3, 3, 4, 2>>(a, st);
-            return launch_stream<Stream<1, 4, 2, 4, 3>>(a, st);
+            if (a->N <= 16) return launch_stream<Stream<1, 1, 5, 5, 4, 2>>(a, st);
+            if (a->N <= 32) return launch_stream<Stream<1, 2, 3, 3, 4, 2>>(a, st);
+            if (narrow_tokens(a->N) == 48) return launch_stream<Stream<1, 3, 3, 3, 4, 2>>(a, st);
+            return launch_stream<Stream<1, 4, 2, 2, 4, 3>>(a, st);
         default:
             if (a->mode == G3K_MV_GEGLU) return launch<Pairs<true>>(a, (a->M[0] + 127) / 128, nb, st);
             return launch<Pairs<false>>(a, row_tiles(a, 256), nb, st);

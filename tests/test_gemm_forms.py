@@ -50,7 +50,7 @@ def test_plan_stays_in_the_launchers_limits(K):
         assert s == 1 or kind == WIDE
 
 
-SHAPES = [(16, 64, 32), (17, 68, 96), (33, 60, 160), (65, 132, 64), (1, 4, 224)]
+SHAPES = [(16, 64, 32), (17, 68, 96), (33, 60, 160), (65, 132, 64), (1, 4, 224), (97, 132, 352)]
 
 
 @pytest.mark.parametrize("cus", [8, 256])   # few and many splits
@@ -72,7 +72,7 @@ def test_many_tokens_on_the_emulated_machine(built, tmp_path):  # noqa: F811
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("N,M,K", SHAPES + [
-    (32, 4, 64), (64, 260, 2592), (128, 2560, 2080), (129, 132, 96), (7, 8, 10240), (48, 2560, 10240),
+    (32, 4, 64), (64, 260, 2592), (77, 2560, 2592), (96, 132, 10240), (128, 2560, 2080), (129, 132, 96), (7, 8, 10240), (48, 2560, 10240),
     (300, 2560, 10240), (1500, 1028, 2592), (4100, 4, 96), (4097, 260, 32)])
 def test_forms(N, M, K):
     rng = np.random.default_rng(N * 7 + M * 13 + K)
@@ -114,7 +114,19 @@ def test_row_lengths(hidden):
     4 and 8 groups of four values per thread): a one-layer batched prefill
     against the token forward over the same tokens, at the 1e-3 x RMS bar of
     the whole-model test (x as two bf16 planes against fp32)."""
-    n, inter, vocab = 17, 64, 96
+    batched_against_token_loop(17, hidden, 64)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,hidden", [(16, 32), (64, 96), (65, 64), (96, 1056), (97, 2080), (128, 96)])
+def test_gate_up_token_classes(n, hidden):
+    """Gate and up as a weight stream at the edges of its token classes (32,
+    64, 96 and 128 per workgroup), from one chunk of K to many."""
+    batched_against_token_loop(n, hidden, 288)
+
+
+def batched_against_token_loop(n, hidden, inter):
+    vocab = 96
     rng = np.random.default_rng(hidden)
 
     def w(*shape, scale):
@@ -129,12 +141,12 @@ def test_row_lengths(hidden):
                  post_feedforward_layernorm=w(hidden, scale=0.1))
     tokens = rng.integers(0, vocab, n).astype(np.int32)
     HW, keep = G.host_weights(w(vocab, hidden, scale=1.0), [layer], w(hidden, scale=0.1))
-    cfg = G.default_config(num_layers=1, hidden_size=hidden, intermediate_size=inter, vocab_size=vocab, max_context=64)
-    with G.Context(cfg, 64) as ctx:
+    cfg = G.default_config(num_layers=1, hidden_size=hidden, intermediate_size=inter, vocab_size=vocab, max_context=max(64, n))
+    with G.Context(cfg, max(64, n)) as ctx:
         ctx.upload_weights(HW)
         got = ctx.prefill_tokens(tokens)
         for i, t in enumerate(tokens):
             want = ctx.forward_token(t, i)
     e = float(np.max(np.abs(got - want)) / np.sqrt(np.mean(want.astype(np.float64) ** 2)))
-    print(f"[rows hidden={hidden}] batched vs token loop {e:.2e}", flush=True)
+    print(f"[rows n={n} hidden={hidden}] batched vs token loop {e:.2e}", flush=True)
     assert e <= 1e-3
