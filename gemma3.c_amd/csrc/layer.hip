@@ -265,9 +265,10 @@ template <int PER, bool VEC>
 __global__ __launch_bounds__(RNT) void rows_kernel(g3k_rows_args a) {
     __shared__ float red[RNW];
     const int row = blockIdx.x, n = a.n, tid = threadIdx.x;
-    if (a.op == G3K_ROWS_SPLIT) {   // elementwise: any row length
+    if (a.op == G3K_ROWS_SPLIT) {   // elementwise: any row length, over gridDim.y workgroups
         const float *t = a.t + (size_t)row * a.ldt;
-        for (int g = tid; 4 * g < n; g += RNT) store_split<VEC>(a, row, g, load4<VEC>(t, g, n));
+        const int step = RNT * gridDim.y;
+        for (int g = tid + RNT * blockIdx.y; 4 * g < n; g += step) store_split<VEC>(a, row, g, load4<VEC>(t, g, n));
         return;
     }
     float *x = a.x + (size_t)row * n;
@@ -337,10 +338,15 @@ __global__ __launch_bounds__(RNT) void rows_kernel(g3k_rows_args a) {
 
 template <int PER>
 void launch_rows(const g3k_rows_args *a, bool vec, hipStream_t st) {
+    // the split has no row sum: a workgroup per 1024 values, so that a few long
+    // rows are one round trip of the whole chip instead of a loop per row (100
+    // rows of 10240 into a projection: the call 30.5 -> 27.9 us)
+    const int parts = a->op == G3K_ROWS_SPLIT ? min((int)((a->n + 4LL * RNT - 1) / (4 * RNT)), 64) : 1;
+    const dim3 grid(a->rows, parts);
     if (vec)
-        hipLaunchKernelGGL((rows_kernel<PER, true>), dim3(a->rows), dim3(RNT), 0, st, *a);
+        hipLaunchKernelGGL((rows_kernel<PER, true>), grid, dim3(RNT), 0, st, *a);
     else
-        hipLaunchKernelGGL((rows_kernel<PER, false>), dim3(a->rows), dim3(RNT), 0, st, *a);
+        hipLaunchKernelGGL((rows_kernel<PER, false>), grid, dim3(RNT), 0, st, *a);
 }
 
 bool aligned(const void *p, size_t b) { return ((uintptr_t)p & (b - 1)) == 0; }

@@ -90,7 +90,7 @@ def test_forms(N, M, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("N,K", [(3, 96), (70, 2592)])
+@pytest.mark.parametrize("N,K", [(3, 96), (70, 2592), (2, 70016)])
 def test_unaligned_activations(N, K):
     """X that is only 4-byte aligned (a slice of a caller's buffer): the split
     into planes falls back to 4-byte loads."""
