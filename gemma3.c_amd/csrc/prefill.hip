@@ -632,9 +632,15 @@ __device__ __forceinline__ void attend(const g3k_prefill_args &p, unsigned char 
 
     // ---- K of the first two tiles and V of the first in flight, then this
     // wave's queries ----
-    fetch_kt(kt0);
-    if (kt0 + 1 <= kt1) fetch_kt(kt0 + 1);
-    fetch_vt(kt0);
+    // A split without tiles fetches none: its kt0 may lie past the staged
+    // rows, and the tile's byte offset is the fetch's scalar offset, which the
+    // range check covers only inside the buffer.  It writes the part of an
+    // empty key range (max NEG_BIG, sum and O zero).
+    if (kt0 <= kt1) {
+        fetch_kt(kt0);
+        if (kt0 + 1 <= kt1) fetch_kt(kt0 + 1);
+        fetch_vt(kt0);
+    }
 
     half8 qh[NQB][8];
     u32x4 qlo[NQB][8];

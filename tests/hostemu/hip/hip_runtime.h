@@ -26,7 +26,10 @@
 //     descriptor's num_records and abort on an out-of-range load instead of
 //     returning zero: the kernels clamp every row index, so none may go out
 //     of range.  Buffer -> LDS loads return zero there, as the hardware
-//     does: the prefill and GEMM kernels rely on it for ragged tiles.
+//     does: the prefill and GEMM kernels rely on it for ragged tiles.  That
+//     check holds only while the scalar offset lies inside the buffer (the
+//     hardware compares the vector offset with num_records minus the scalar
+//     one, which wraps), so a scalar offset past num_records aborts.
 //   - MFMA 16x16x32 (f16 / bf16) computes the exact products and sums them
 //     in double: any operand placed in the wrong lane changes the result.
 //   - DPP controls and load forms other than the ones the kernels use abort.
@@ -315,10 +318,16 @@ inline __amdgpu_buffer_rsrc_t hostemu_make_buffer_rsrc(void *base, short stride,
     (void)flags;
     return __amdgpu_buffer_rsrc_t{static_cast<const char *>(base), (uint32_t)num_records};
 }
+// The byte offset of a buffer access; a scalar offset past the buffer's end,
+// where the hardware's range check no longer holds, aborts.
+inline uint64_t hostemu_buffer_offset(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff) {
+    if (soff > r.num_records) hostemu::fail("buffer access with a scalar offset beyond num_records");
+    return (uint64_t)voff + soff;
+}
 inline std::array<uint32_t, 4> hostemu_raw_buffer_load_b128(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff,
                                                            int aux) {
     (void)aux;
-    const uint64_t off = (uint64_t)voff + soff;
+    const uint64_t off = hostemu_buffer_offset(r, voff, soff);
     if (off + 16 > r.num_records) hostemu::fail("buffer load beyond num_records");
     std::array<uint32_t, 4> v;
     std::memcpy(v.data(), r.base + off, 16);
@@ -329,14 +338,14 @@ template <typename T>
 inline void hostemu_raw_buffer_store_b128(T v, __amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff, int aux) {
     static_assert(sizeof(T) == 16, "b128 store");
     (void)aux;
-    const uint64_t off = (uint64_t)voff + soff;
+    const uint64_t off = hostemu_buffer_offset(r, voff, soff);
     if (off + 16 > r.num_records) hostemu::fail("buffer store beyond num_records");
     std::memcpy(const_cast<char *>(r.base) + off, &v, 16);
 }
 // 4- and 8-byte buffer loads into registers, range-checked like the b128 form.
 inline uint32_t hostemu_raw_buffer_load_b32(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff, int aux) {
     (void)aux;
-    const uint64_t off = (uint64_t)voff + soff;
+    const uint64_t off = hostemu_buffer_offset(r, voff, soff);
     if (off + 4 > r.num_records) hostemu::fail("buffer load beyond num_records");
     uint32_t v;
     std::memcpy(&v, r.base + off, 4);
@@ -345,7 +354,7 @@ inline uint32_t hostemu_raw_buffer_load_b32(__amdgpu_buffer_rsrc_t r, unsigned v
 inline std::array<uint32_t, 2> hostemu_raw_buffer_load_b64(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff,
                                                           int aux) {
     (void)aux;
-    const uint64_t off = (uint64_t)voff + soff;
+    const uint64_t off = hostemu_buffer_offset(r, voff, soff);
     if (off + 8 > r.num_records) hostemu::fail("buffer load beyond num_records");
     std::array<uint32_t, 2> v;
     std::memcpy(v.data(), r.base + off, 8);
@@ -368,8 +377,9 @@ inline void hostemu_buffer_load_lds(__amdgpu_buffer_rsrc_t r, P lds, int size, u
     (void)aux;
     if ((size != 16 && size != 4) || offset != 0) hostemu::fail("buffer->LDS load form not emulated");
     char *dst = (char *)lds + size * hostemu::t_lane;
+    const uint64_t off = hostemu_buffer_offset(r, voff, soff);
     for (int i = 0; i < size / 4; i++) {
-        const uint64_t o = (uint64_t)voff + soff + 4 * i;
+        const uint64_t o = off + 4 * i;
         uint32_t v = 0;
         if (o + 4 <= r.num_records) std::memcpy(&v, r.base + o, 4);
         std::memcpy(dst + 4 * i, &v, 4);

@@ -18,6 +18,17 @@ def test_forced_on_the_emulated_machine(built, tmp_path, splits):  # noqa: F811
     assert launches["prefill_merge_kernel"][0] == 2, launches
 
 
+def test_the_rules_empty_splits_fetch_nothing_out_of_range(built, tmp_path):  # noqa: F811
+    """16 tokens at position 2035 are 65 key tiles, which the rule deals to 16
+    splits five at a time: three of them get none.  The emulated machine stops
+    a buffer access whose scalar offset passes the buffer's end."""
+    e = Emu(tmp_path, H=1, Hkv=1, max_context=2056, window=64)
+    e.kv_append(5, 0, 2035)
+    e.prefill(5, 2035, 16)
+    launches = e.run()
+    assert launches["prefill_kernel"] == (1, 16) and launches["prefill_merge_kernel"][0] == 1, launches
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("splits", [8, 16])
 def test_forced_split_counts(monkeypatch, splits):
