@@ -327,10 +327,16 @@ __device__ __forceinline__ void Stream<MT, NTL, DW, DX, NWV, OCC>::run(const g3k
     };
     // The rings' waits count fetches in issue order, so no round may move
     // into another: a scheduling fence after each.  The round of chunk c
-    // fetches x of chunk c + DX - 1, then W of chunk c + DW - 1.
+    // fetches x of chunk c + DX - 1, then W of chunk c + DW - 1.  With DW >
+    // DX the wait for chunk c leaves the W fetched after its x in flight, so
+    // there a round's x comes before its W: a fence between them too.
+    auto x_first = [] {
+        if (DW > DX) G3K_ORDER_FENCE();
+    };
 #pragma unroll
     for (int d = 1 - DW; d < 0; d++) {
         if (d + DX - 1 >= 0) fetch_x(d + DX - 1, c0 + d + DX - 1);
+        x_first();
         fetch_w(d + DW - 1, c0 + d + DW - 1);
         G3K_ORDER_FENCE();
     }
@@ -342,6 +348,7 @@ __device__ __forceinline__ void Stream<MT, NTL, DW, DX, NWV, OCC>::run(const g3k
         // whose slots are filled next
         G3K_WAIT_BARRIER((DX - 2) * (NWI + NXI) + (DW > DX ? NWI : 0));
         fetch_x(sx == 0 ? DX - 1 : sx - 1, c + DX - 1);
+        x_first();
         fetch_w(sw == 0 ? DW - 1 : sw - 1, c + DW - 1);
         G3K_ORDER_FENCE();
         const char *ws = smem + sw * W_B + wave * (MT * 2048), *xs = smem + DW * W_B + sx * (2 * X_B);

@@ -17,6 +17,9 @@
 //   prefill_device ...                          (same, device pointers)
 //   decode layer pos q k v q_norm k_norm out
 //   matmul N M K W X C                          (g3attn_matmul_bf16_device)
+//   gemm kind ksplit geglu N M K W0 W1|- xh xl out   (g3k_gemm as asked: W1 the
+//                    up matrix with geglu = 1; out fp32 [N][M], with geglu
+//                    the sum of the two bf16 planes; split sums through part)
 //   gqa H Hkv seq q k v mask|- out [head_dim]   (g3attn_gqa, host pointers;
 //                                                head_dim 256 if absent, scale
 //                                                1 / sqrt(head_dim))
@@ -261,6 +264,63 @@ int main(int argc, char **argv) {
             hipFree(dX);
             hipFree(dC);
             write_bin(cf, C.data(), C.size());
+        } else if (cmd == "gemm") {
+            int kind, S, geglu, N, M, K;
+            std::string w0, w1, hf, lf, of;
+            in >> kind >> S >> geglu >> N >> M >> K >> w0 >> w1 >> hf >> lf >> of;
+            if (!in) die("bad gemm line");
+            const size_t nm = (size_t)N * M;
+            std::vector<uint16_t *> dev = {to_device(read_bin<uint16_t>(w0, (size_t)M * K)),
+                                           to_device(read_bin<uint16_t>(hf, (size_t)N * K)),
+                                           to_device(read_bin<uint16_t>(lf, (size_t)N * K)),
+                                           to_device(std::vector<uint16_t>(nm, 0x7fff)),
+                                           to_device(std::vector<uint16_t>(nm, 0x7fff))};
+            if (geglu) dev.push_back(to_device(read_bin<uint16_t>(w1, (size_t)M * K)));
+            std::vector<float> C(nm, -12345.0f);
+            float *dC = to_device(C), *part = nullptr;
+            const bool tile = kind == G3K_GEMM_TILE;
+            if (S > 1 || (geglu && !tile)) part = to_device(std::vector<float>(S * nm * (geglu ? 2 : 1), -12345.0f));
+            g3k_gemm_args g;
+            std::memset(&g, 0, sizeof g);
+            g.x_hi = dev[1];
+            g.x_lo = dev[2];
+            g.N = N;
+            g.K = K;
+            g.ldx = K;
+            g.n_mat = geglu ? 2 : 1;
+            g.mode = geglu ? G3K_MV_GEGLU : 0;
+            g.kind = kind;
+            g.ksplit = S;
+            g.W[0] = dev[0];
+            g.M[0] = M;
+            if (geglu) {
+                g.W[1] = dev[5];
+                g.M[1] = M;
+                g.h_hi = dev[3];
+                g.h_lo = dev[4];
+                g.ldh = M;
+            } else {
+                g.C[0] = dC;
+                g.ldc[0] = M;
+            }
+            g.part = part;
+            const int rc = g3k_gemm(&g, nullptr);
+            if (rc) die("g3k_gemm returned " + std::to_string(rc));
+            if (geglu) {
+                for (size_t i = 0; i < nm; i++) {
+                    const uint32_t h = (uint32_t)dev[3][i] << 16, l = (uint32_t)dev[4][i] << 16;
+                    float fh, fl;
+                    std::memcpy(&fh, &h, 4);
+                    std::memcpy(&fl, &l, 4);
+                    C[i] = fh + fl;
+                }
+            } else {
+                hipMemcpy(C.data(), dC, nm * sizeof(float), hipMemcpyDeviceToHost);
+            }
+            for (uint16_t *p : dev) hipFree(p);
+            hipFree(dC);
+            hipFree(part);
+            write_bin(of, C.data(), nm);
         } else if (cmd == "gqa" || cmd == "gqa_noalloc") {
             int h, hkv, seq, hd = (int)D;
             std::string qf, kf, vf, mf, of;

@@ -21,7 +21,14 @@
 //     waves of a workgroup interleave at every cross-lane step.
 //   - Loads complete when issued: a buffer -> LDS fetch writes LDS at once,
 //     so one that overwrites data another wave still reads (a missing
-//     barrier) shows in the results.
+//     barrier) shows in the results.  With HOSTEMU_FETCH=late it completes
+//     only where the kernel waits for it (G3K_WAIT_VMEM, __syncthreads, or a
+//     G3K_WAIT_BARRIER that does not leave it in flight), so a read ahead of
+//     its wait shows instead.  In both modes a G3K_WAIT_BARRIER aborts where
+//     the fetches it leaves in flight and the ones it waits for were issued
+//     with nothing between them that fixes their order (G3K_ORDER_FENCE or a
+//     wait): there the compiler may issue them in another order than the
+//     count assumes.
 //   - Buffer loads into registers check their offset against the
 //     descriptor's num_records and abort on an out-of-range load instead of
 //     returning zero: the kernels clamp every row index, so none may go out
@@ -89,11 +96,10 @@ inline float __int_as_float(int u) { float f; std::memcpy(&f, &u, 4); return f; 
 template <typename K>
 hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, K, int, size_t) { *n = 2; return hipSuccess; }
 
-// Loads complete when issued here, so the library's explicit wait for them
-// is empty.
-#define G3K_WAIT_VMEM() ((void)0)
-#define G3K_WAIT_BARRIER(n) __syncthreads()
-#define G3K_ORDER_FENCE() ((void)0)
+// The library's explicit waits for buffer -> LDS fetches (see the top).
+#define G3K_WAIT_VMEM() hostemu::complete_fetches(0)
+#define G3K_WAIT_BARRIER(n) (hostemu::complete_fetches(n), hostemu::machine()->block.wait())
+#define G3K_ORDER_FENCE() ((void)hostemu::machine()->current->fence++)
 // The emulated machine deals workgroup i to XCD i mod 8, as the MI355X
 // dispatcher does.
 #define G3K_XCC_ID() (blockIdx.x % 8u)
@@ -119,7 +125,17 @@ namespace hostemu {
     std::abort();
 }
 
+// A buffer -> LDS fetch of one lane that the kernel has not waited for yet.
+struct Fetch {
+    char *dst;
+    uint32_t v[4];
+    int size;
+    unsigned fence;           // the lane's order fences before it
+};
+
 struct Fiber {
+    std::vector<Fetch> fetches;   // in issue order
+    unsigned fence = 0;
     void *sp = nullptr;       // saved stack pointer while switched out
     char *stack = nullptr;
     size_t stack_size = 0;
@@ -160,8 +176,30 @@ struct Machine {
     std::function<void()> body;
 };
 
+inline bool late_fetches() {
+    static const bool late = [] {
+        const char *e = std::getenv("HOSTEMU_FETCH");
+        return e && !std::strcmp(e, "late");
+    }();
+    return late;
+}
+
 inline Machine *&machine() { static Machine *m = nullptr; return m; }
 inline int t_lane = 0, t_wave = 0, t_flat = 0;
+
+// Completes all of the running lane's fetches but the youngest n.
+inline void complete_fetches(int n) {
+    Fiber &f = *machine()->current;
+    const int done = (int)f.fetches.size() - n;
+    if (done > 0) {
+        if (n > 0 && f.fetches[done - 1].fence == f.fetches[done].fence)
+            fail("a counted wait splits fetches whose issue order nothing fixes");
+        if (late_fetches())
+            for (int i = 0; i < done; i++) std::memcpy(f.fetches[i].dst, f.fetches[i].v, f.fetches[i].size);
+        f.fetches.erase(f.fetches.begin(), f.fetches.begin() + done);
+    }
+    f.fence++;
+}
 
 // Switches from the running fiber back to the scheduler.
 inline void yield_to_scheduler(bool dying) {
@@ -205,7 +243,10 @@ inline void exchange(uint32_t x, uint32_t y, int src, uint32_t *rx, uint32_t *ry
 }  // namespace hostemu
 
 inline dim3 threadIdx, blockIdx, gridDim, blockDim;
-inline void __syncthreads() { hostemu::machine()->block.wait(); }
+inline void __syncthreads() {
+    hostemu::complete_fetches(0);
+    hostemu::machine()->block.wait();
+}
 // Barrier that also returns whether any thread of the workgroup passed nonzero.
 inline int __syncthreads_or(int p) {
     hostemu::Machine &m = *hostemu::machine();
@@ -378,12 +419,15 @@ inline void hostemu_buffer_load_lds(__amdgpu_buffer_rsrc_t r, P lds, int size, u
     if ((size != 16 && size != 4) || offset != 0) hostemu::fail("buffer->LDS load form not emulated");
     char *dst = (char *)lds + size * hostemu::t_lane;
     const uint64_t off = hostemu_buffer_offset(r, voff, soff);
+    hostemu::Fetch f{dst, {}, size, hostemu::machine()->current->fence};
     for (int i = 0; i < size / 4; i++) {
         const uint64_t o = off + 4 * i;
         uint32_t v = 0;
         if (o + 4 <= r.num_records) std::memcpy(&v, r.base + o, 4);
-        std::memcpy(dst + 4 * i, &v, 4);
+        f.v[i] = v;
     }
+    if (!hostemu::late_fetches()) std::memcpy(dst, f.v, size);
+    hostemu::machine()->current->fetches.push_back(f);
 }
 #define __builtin_amdgcn_raw_ptr_buffer_load_lds hostemu_buffer_load_lds
 

@@ -70,6 +70,49 @@ def test_many_tokens_on_the_emulated_machine(built, tmp_path):  # noqa: F811
     e.run()
 
 
+def emu_gemm(e, kind, ksplit, geglu, N, M, K):
+    """One g3k_gemm of a given form on the emulated machine, against fp64."""
+    W = [(e.rng.standard_normal((M, K)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16) for _ in range(1 + geglu)]
+    X = (e.rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32)
+    hi = (X.view(np.uint32) & 0xFFFF0000).view(np.float32)
+    lo = ((X - hi).view(np.uint32) & 0xFFFF0000).view(np.float32)
+    files = [e._name(f) for f in ("W", "U", "xh", "xl", "C")]
+    e._save(files[0], W[0])
+    if geglu:
+        e._save(files[1], W[1])
+    e._save(files[2], (hi.view(np.uint32) >> 16).astype(np.uint16))
+    e._save(files[3], (lo.view(np.uint32) >> 16).astype(np.uint16))
+    e.lines.append(f"gemm {kind} {ksplit} {geglu} {N} {M} {K} " + " ".join(files))
+    X64 = hi.astype(np.float64) + lo
+    W64 = [(w.astype(np.uint32) << 16).view(np.float32).astype(np.float64) for w in W]
+    # fp32 accumulation of the planes' exact products, in any order
+    prod, bound = [X64 @ w.T for w in W64], [2 * K * 2.0 ** -24 * (np.abs(X64) @ np.abs(w).T) + 1e-30 for w in W64]
+    want, bar = prod[0], bound[0]
+    if geglu:
+        g, u = prod
+        gelu = 0.5 * g * (1 + np.tanh(0.7978845608028654 * (g + 0.044715 * g ** 3)))
+        want = gelu * u
+        # |gelu'| <= 1.13; gelu and the product in fp32; the planes' 2^-16
+        bar = 1.13 * bound[0] * (np.abs(u) + bound[1]) + np.abs(gelu) * bound[1]
+        bar = bar + 2.0 ** -16 * np.abs(want) + 8 * 2.0 ** -24 * np.abs(g * u)
+    e.checks.append((files[4], want, f"gemm kind={kind} S={ksplit} geglu={geglu} N={N} M={M} K={K}", bar))
+
+
+@pytest.mark.parametrize("fetch", ["early", "late"])
+@pytest.mark.parametrize("kind,geglu,N", [(WIDE, 1, n) for n in (32, 64, 96, 128)]
+                         + [(NARROW, 0, n) for n in (16, 32, 48, 64)] + [(TILE, 0, 128), (TILE, 1, 128)])
+def test_rings_turn_over(built, tmp_path, kind, geglu, N, fetch):  # noqa: F811
+    """Each form with more chunks per split than its LDS rings have slots, so
+    that every slot is refilled while others are read: 11 and 12 chunks (the
+    last a half one) in two splits, the tiles' gate and up 23 in one.  Late:
+    a fetch lands where the kernel waits for it and no earlier, so a count
+    that waits for one too few reads the slot's old chunk; and a counted wait
+    may only split fetches whose issue order is fixed."""
+    e = Emu(tmp_path)
+    emu_gemm(e, kind, 1 if kind == TILE and geglu else 2, geglu, N, 60, 22 * 64 + 32)
+    e.run(HOSTEMU_FETCH=fetch)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("N,M,K", SHAPES + [
     (32, 4, 64), (64, 260, 2592), (77, 2560, 2592), (96, 132, 10240), (128, 2560, 2080), (129, 132, 96), (7, 8, 10240), (48, 2560, 10240),
