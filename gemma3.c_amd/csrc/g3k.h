@@ -273,6 +273,10 @@ typedef struct {
 
 int g3k_matvec(const g3k_matvec_args *a, void *stream);
 
+/* Whether the residual prologue costs this launch (its mode, A, M and K) less
+ * than a launch of its own. */
+int g3k_matvec_prologue_pays(const g3k_matvec_args *a);
+
 /* One-workgroup steps of a token's forward pass on a hidden vector of n
  * floats (n <= G3K_LAYER_MAX_HIDDEN):
  *   G3K_OP_EMBED:    x = bf16(embed[token][.]) * sqrt(n)

@@ -444,6 +444,28 @@ hipError_t launch(const g3k_matvec_args *a, hipStream_t st) {
 
 }  // namespace
 
+namespace {
+
+// The vector path reads rows in 16-byte chunks and addresses each matrix
+// through a 32-bit byte offset.
+bool vector_path(const g3k_matvec_args *a) {
+    bool vec = a->K % 8 == 0;
+    for (int m = 0; m < a->n_mat; m++)
+        vec = vec && ((uintptr_t)a->A[m] & 15) == 0 && (long long)a->M[m] * a->K * 2 < (1LL << 32);
+    return vec;
+}
+
+}  // namespace
+
+// The resident form runs the prologue once per workgroup of 512.  The scalar
+// GEGLU launch runs it once per two rows: up to one round of eight workgroups
+// per CU that costs less than the step's own launch, beyond it more (18
+// layers, us a token, own launch against prologue: hidden 644, intermediate
+// 2048: 574 / 549; 1156, 6912: 873 / 899; 2564, 10240: 1484 / 1553).
+extern "C" int g3k_matvec_prologue_pays(const g3k_matvec_args *a) {
+    return a->mode != G3K_MV_GEGLU || vector_path(a) || a->M[0] <= 2 * 2048;
+}
+
 extern "C" int g3k_matvec(const g3k_matvec_args *a, void *stream) {
     const bool pre = a->pre_t != nullptr;
     if (a->n_mat < 1 || a->n_mat > G3K_MATVEC_MAX || a->K < 1 || (!pre && !a->x))
@@ -455,18 +477,15 @@ extern "C" int g3k_matvec(const g3k_matvec_args *a, void *stream) {
                  (uintptr_t)a->pre_r < (uintptr_t)(a->pre_r_out + a->K))))
         return (int)hipErrorInvalidValue;
     // with the prologue x comes from LDS, 16-byte aligned
-    bool vec = a->K % 8 == 0 && (pre || ((uintptr_t)a->x & 15) == 0);
+    const bool vec = (pre || ((uintptr_t)a->x & 15) == 0) && vector_path(a);
     long long rows = 0;
     for (int m = 0; m < a->n_mat; m++) {
         // GEGLU writes one output (y[0]) from the two matrices
         if (a->M[m] < 1 || !a->A[m] || (!a->y[m] && (a->mode != G3K_MV_GEGLU || m == 0)))
             return (int)hipErrorInvalidValue;
-        vec = vec && ((uintptr_t)a->A[m] & 15) == 0;
         rows += a->M[m];
     }
     if (rows > (1LL << 30)) return (int)hipErrorInvalidValue;
-    // the vector path addresses each matrix through a 32-bit byte offset
-    for (int m = 0; m < a->n_mat; m++) vec = vec && (long long)a->M[m] * a->K * 2 < (1LL << 32);
     hipStream_t st = (hipStream_t)stream;
     if (a->mode == G3K_MV_GEGLU) {
         if (a->n_mat != 2 || a->M[0] != a->M[1]) return (int)hipErrorInvalidValue;

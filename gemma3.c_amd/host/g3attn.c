@@ -1380,7 +1380,8 @@ static int forward_enqueue(g3attn_ctx *c, const g3attn_weights *w, int token_id,
         if ((rc = gemv(c, proj, lw->o_proj, attn, hid, qs))) return rc;
         /* layer_mlp (:480-487, 369-388): gate and up GEMVs with gelu(gate) * up,
          * after the post-attention norm, residual add and pre-feedforward
-         * norm (:463-477), folded into the launch's prologue with fold_mlp */
+         * norm (:463-477), folded into the launch's prologue with fold_mlp
+         * where that pays */
         g3k_matvec_args a;
         memset(&a, 0, sizeof a);
         a.K = hid;
@@ -1390,7 +1391,8 @@ static int forward_enqueue(g3attn_ctx *c, const g3attn_weights *w, int token_id,
         a.A[1] = lw->up_proj;
         a.y[0] = h;
         a.M[0] = a.M[1] = inter;
-        if (fold_mlp && AL8(lw->post_attention_layernorm) && AL8(lw->pre_feedforward_layernorm)) {
+        if (fold_mlp && g3k_matvec_prologue_pays(&a) && AL8(lw->post_attention_layernorm) &&
+            AL8(lw->pre_feedforward_layernorm)) {
             set_pre(&a, cfg, &x, &x_alt, proj, lw->post_attention_layernorm, lw->pre_feedforward_layernorm);
         } else {
             if ((rc = layer_step(c, G3K_OP_RESIDUAL, x, proj, xn, lw->post_attention_layernorm,

@@ -469,8 +469,8 @@ def test_random_sessions(built, tmp_path, seed):
 SMALL = dict(hidden=128, inter=256, vocab=256, layers=6, max_context=32, window=8, heads=2, kv_heads=1)
 
 
-def _forward_model(n):
-    f = SMALL
+def _forward_model(n, **dims):
+    f = dict(SMALL, **dims)
     cfg = O.Config(num_layers=f["layers"], max_context=f["max_context"], sliding_window=f["window"],
                    num_heads=f["heads"], num_kv_heads=f["kv_heads"])
     Hd, I, V = f["hidden"], f["inter"], f["vocab"]
@@ -526,6 +526,22 @@ def test_token_forward(built, tmp_path, fold):
         e.logits("forward_device", f"{int(t)} {i}", want[i], f"forward_device token {i} fold={fold}")
     launches = e.run(G3ATTN_FORWARD_FOLD=fold)
     assert launches["residual_kernel"][0] == n * RESIDUAL_PER_TOKEN[fold], launches
+
+
+@pytest.mark.parametrize("hidden,inter,per_token", [(132, 256, 1), (132, 4100, 3), (128, 4100, 1)])
+def test_fold_of_the_scalar_gate_up(built, tmp_path, hidden, inter, per_token):
+    """A hidden size that is no multiple of 8 puts the gate/up launch on the
+    scalar path, where every two rows repeat the residual step: by default
+    that step is folded up to 2048 workgroups and stays a kernel beyond (the
+    one before each Q/K/V launch is folded as before).  Two layers: three
+    residual kernels a token without the gate/up fold, one with it."""
+    f, embed, layers, norm, tokens, want = _forward_model(2, hidden=hidden, inter=inter, layers=2)
+    e = _emu_for(tmp_path, f)
+    e.model(embed, layers, norm)
+    for i, t in enumerate(tokens):
+        e.logits("forward_device", f"{int(t)} {i}", want[i], f"forward_device token {i} hidden {hidden} inter {inter}")
+    launches = e.run()
+    assert launches["residual_kernel"][0] == 2 * per_token, launches
 
 
 def test_upload_batched_prefill_then_decode(built, tmp_path):
