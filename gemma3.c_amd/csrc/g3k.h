@@ -329,15 +329,16 @@ int g3k_rows(const g3k_rows_args *a, void *stream);
  * M % 4 == 0).  mode 0: n_mat (1..3) matrices sharing X, each written to C[j]
  * [N][ldc[j]] fp32.  mode G3K_MV_GEGLU: W[0] = gate, W[1] = up (same M);
  * gelu_tanh(gate) * up is written as bf16 planes h_hi + h_lo [N][ldh].
- * kind: G3K_GEMM_TILE, 256 weight rows x 128 tokens per workgroup; _WIDE and
- * _NARROW, few tokens, 256 and 64 rows.
+ * kind: G3K_GEMM_TILE, 256 weight rows x 128 tokens per workgroup; _QUAD128
+ * and _QUAD256 (plain), 128 and 256 rows x 128 tokens, two workgroups per CU;
+ * _WIDE and _NARROW, few tokens, 256 and 64 rows.
  * ksplit S > 1 (plain, or GEGLU of _WIDE / _NARROW): split s sums its share of
  * the 64-wide chunks of k.  With part [S][N][sum of M] the partial products
  * go there and a second launch adds them in split order (GEGLU of _WIDE /
  * _NARROW: required); without it they go to C[j] + s * split_stride
  * (floats), for the consumer to add.  g3k_gemm_plan picks kind and ksplit
  * (consumer_adds: the partial products go to C). */
-enum { G3K_GEMM_TILE = 0, G3K_GEMM_WIDE = 1, G3K_GEMM_NARROW = 2 };
+enum { G3K_GEMM_TILE = 0, G3K_GEMM_WIDE = 1, G3K_GEMM_NARROW = 2, G3K_GEMM_QUAD128 = 3, G3K_GEMM_QUAD256 = 4 };
 void g3k_gemm_plan(int N, int K, int n_mat, const int *M, int geglu, int consumer_adds, int n_cu, int *kind,
                    int *ksplit);
 typedef struct {

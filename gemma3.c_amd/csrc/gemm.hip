@@ -12,10 +12,10 @@
 // with fp32 accumulation: twice the algorithmic MFMA work, within a few
 // 2^-17 of the reference's fp32 sgemm.
 //
-// Tiling.  Two forms of gemm_kernel, picked by g3k_gemm_plan: Pairs (many
-// tokens) and Stream in two widths (few tokens); each says what bounds it.  In
-// both W and x tiles move
-// from global memory straight into LDS with buffer -> LDS loads
+// Tiling.  Three forms of gemm_kernel, picked by g3k_gemm_plan: Pairs (many
+// tokens), Quads (many tokens, short rows) and Stream in two widths (few
+// tokens); each says what bounds it.  In all of them W and x tiles move from
+// global memory straight into LDS with buffer -> LDS loads
 // (buffer_load_dwordx4 ... lds, one wave instruction = 1 KiB).  Rows beyond M
 // or N read zero (the buffer descriptor's range check), so ragged tiles need
 // no masking until the stores.  A row's 16-byte pieces are XOR-swizzled by
@@ -244,6 +244,106 @@ __device__ __forceinline__ void Pairs<GEGLU>::run(const g3k_gemm_args &a) {
 }
 
 // ---------------------------------------------------------------------------
+// Short rows (K up to about 2000), or grids of tiles that leave a last round
+// nearly empty: 32 MT weight rows x 128 tokens (MT = 4, 8) per workgroup of 4
+// waves, a quarter of the tile each, two workgroups per CU, K in stages of 32.
+// One's first fetches and last stores (a whole output tile of 64 or 128 KiB)
+// run under the other's K loop; with one workgroup per CU, as in Pairs, they
+// add to it.  Against Pairs at S = 1 (us): 1024 tokens, 102400 x 96: 149 ->
+// 115; 2048 tokens, 12368 x 352: 68 -> 56; 1024, 10240 x 512: 35.0 -> 30.8;
+// 2048, 10240 x 2560: 189 -> 202.
+// LDS rows are 64 B; within each 16-row group the four 16-byte pieces of row
+// r sit at slot 4 r + (c ^ (r / 4 % 4)), so a fragment read (16 rows, one
+// piece) touches all 64 banks once.
+template <int MT>
+struct Quads {
+    static constexpr int THREADS = 256, WAVES = 2, ROWS = 32 * MT, TOKENS = BN;
+    static constexpr int PART_B = 128 * BK * 2;   // 128 rows of a stage: 8 KiB
+    // Rows row0 .. row0 + 127, k0 .. k0 + 31 of a [rows][ld] matrix into LDS:
+    // wave w takes the 16-row groups w and w + 4, lane i slot i of a group.
+    static __device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t rs, char *dst, int row0, int ld, int k0,
+                                                 int wave, int lane) {
+        const int r = lane >> 2, c = (lane & 3) ^ ((r >> 2) & 3);
+#pragma unroll
+        for (int g = wave; g < 8; g += 4)
+            fetch8(rs, dst + g * 1024, (uint32_t)(row0 + g * 16 + r) * (uint32_t)ld * 2u + c * 16, (uint32_t)k0 * 2u);
+    }
+    static __device__ __forceinline__ bf16x8 frag(const char *st, int r, int c) {
+        return *reinterpret_cast<const bf16x8 *>(st + ((r >> 4) * 64 + (r & 15) * 4 + (c ^ ((r >> 2) & 3))) * 16);
+    }
+    static __device__ void run(const g3k_gemm_args &a);
+};
+template <int MT>
+__device__ __forceinline__ void Quads<MT>::run(const g3k_gemm_args &a) {
+    constexpr int W_B = ROWS * BK * 2, STAGE_B = W_B + 2 * PART_B;
+    __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE_B];
+    int bx = blockIdx.x, m_idx = 0;
+    while (m_idx + 1 < a.n_mat && bx >= (a.M[m_idx] + ROWS - 1) / ROWS) {
+        bx -= (a.M[m_idx] + ROWS - 1) / ROWS;
+        m_idx++;
+    }
+    const int M = a.M[m_idx], K = a.K, N = a.N;
+    const int m0 = bx * ROWS, n0 = blockIdx.y * BN;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave & 1, wn = wave >> 1;
+    const int fr = lane & 15, fc = lane >> 4;
+    const __amdgpu_buffer_rsrc_t rw = rsrc(a.W[m_idx], (uint32_t)((size_t)M * K * 2));
+    const uint32_t xbytes = (uint32_t)((size_t)N * a.ldx * 2);
+    const __amdgpu_buffer_rsrc_t rxh = rsrc(a.x_hi, xbytes), rxl = rsrc(a.x_lo, xbytes);
+
+    f32x4 acc[MT][4];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nt = 0; nt < 4; nt++) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto fetch_stage = [&](int s, int k0) {
+        char *st = smem + s * STAGE_B;
+#pragma unroll
+        for (int h = 0; h < ROWS / 128; h++) fetch(rw, st + h * PART_B, m0 + 128 * h, K, k0, wave, lane);
+        fetch(rxh, st + W_B, n0, a.ldx, k0, wave, lane);
+        fetch(rxl, st + W_B + PART_B, n0, a.ldx, k0, wave, lane);
+    };
+    // split z takes stages [t0, t1) of 32 k values
+    const int stages = K / BK;
+    const int t0 = (int)((long long)stages * blockIdx.z / a.ksplit);
+    const int t1 = (int)((long long)stages * (blockIdx.z + 1) / a.ksplit);
+    fetch_stage(0, t0 * BK);
+    for (int t = t0; t < t1; t++) {
+        const int s = (t - t0) & 1;
+        __syncthreads();   // stage t has landed; the other slot is free
+        if (t + 1 < t1) fetch_stage(s ^ 1, (t + 1) * BK);
+        const char *st = smem + s * STAGE_B;
+        bf16x8 h[4], l[4];
+#pragma unroll
+        for (int nt = 0; nt < 4; nt++) {
+            h[nt] = frag(st + W_B, wn * 64 + nt * 16 + fr, fc);
+            l[nt] = frag(st + W_B + PART_B, wn * 64 + nt * 16 + fr, fc);
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            const bf16x8 w = frag(st, wm * 16 * MT + mt * 16 + fr, fc);
+#pragma unroll
+            for (int nt = 0; nt < 4; nt++) {
+                acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, h[nt], acc[mt][nt], 0, 0, 0);
+                acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, l[nt], acc[mt][nt], 0, 0, 0);
+            }
+        }
+    }
+    // lane holds rows m = base + 4 (l / 16) + i, i = 0..3, of token l % 16
+    long long ld;
+    float *C = out_base(a, m_idx, blockIdx.z, ld);
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nt = 0; nt < 4; nt++) {
+            const int m = m0 + wm * 16 * MT + mt * 16 + 4 * fc, n = n0 + wn * 64 + nt * 16 + fr;
+            if (n >= N || m >= M) continue;   // M is a multiple of 4 (checked on the host)
+            const f32x4 c = acc[mt][nt];
+            *reinterpret_cast<float4 *>(C + (size_t)n * ld + m) = make_float4(c[0], c[1], c[2], c[3]);
+        }
+}
+
+// ---------------------------------------------------------------------------
 // Few tokens: the weight stream.
 //
 // With N <= 128 tokens (a short message, a ragged tail) the projection is one
@@ -391,7 +491,7 @@ __device__ __forceinline__ void Stream<MT, NTL, DW, DX, NWV, OCC>::run(const g3k
         }
 }
 
-// One launch of form F (Stream, Pairs).
+// One launch of form F (Stream, Pairs, Quads).
 template <class F>
 __global__ __launch_bounds__(F::THREADS, F::WAVES) void gemm_kernel(g3k_gemm_args a) {
     F::run(a);
@@ -476,6 +576,10 @@ int launch_form(const g3k_gemm_args *a, hipStream_t st) {
             if (a->N <= 32) return launch_stream<Stream<1, 2, 3, 3, 4, 2>>(a, st);
             if (narrow_tokens(a->N) == 48) return launch_stream<Stream<1, 3, 3, 3, 4, 2>>(a, st);
             return launch_stream<Stream<1, 4, 2, 2, 4, 3>>(a, st);
+        case G3K_GEMM_QUAD128:
+            return launch_stream<Quads<4>>(a, st);
+        case G3K_GEMM_QUAD256:
+            return launch_stream<Quads<8>>(a, st);
         default:
             if (a->mode == G3K_MV_GEGLU) return launch<Pairs<true>>(a, (a->M[0] + 127) / 128, nb, st);
             return launch<Pairs<false>>(a, row_tiles(a, 256), nb, st);
@@ -484,17 +588,70 @@ int launch_form(const g3k_gemm_args *a, hipStream_t st) {
 
 }  // namespace
 
+namespace {
+
+// A form's time, in us at 256 CUs, as fitted to 5500 measured products (N 1 to
+// 4097, M 4 to 262208, K 32 to 10240; each form within 5 to 12% rms):
+//   2.3 + rounds (round + chunk[o - 1] chunks) + w_read W MB per token block
+//   + out C MB (+ 3.3 + 0.32 S C MB for split sums that a second launch adds)
+// A round is per_cu workgroups on every CU; o, how many share a CU in it.
+// tokens: the most a row of the table holds for (Stream's token classes).
+struct FormTime {
+    int kind, rows, tokens, per_cu;
+    double round, chunk[3], w_read, out;
+};
+constexpr FormTime FORMS[] = {
+    {G3K_GEMM_NARROW, 64, 16, 2, 0.68, {0.18, 0.50, 0}, 0.044, 0.178},
+    {G3K_GEMM_NARROW, 64, 32, 2, 0.54, {0.30, 0.55, 0}, 0.049, 0.084},
+    {G3K_GEMM_NARROW, 64, 48, 2, 0.62, {0.30, 0.55, 0}, 0.051, 0.150},
+    {G3K_GEMM_NARROW, 64, 64, 3, 0.59, {0.42, 0.49, 0.73}, 0.075, 0.108},
+    {G3K_GEMM_WIDE, 256, 64, 1, 0.85, {0.67, 0, 0}, 0.111, 0.214},
+    {G3K_GEMM_WIDE, 256, 96, 1, 1.17, {0.99, 0, 0}, 0.078, 0.227},
+    {G3K_GEMM_WIDE, 256, 128, 1, 1.92, {1.34, 0, 0}, 0.059, 0.197},
+    {G3K_GEMM_TILE, 256, 128, 1, 2.19, {1.23, 0, 0}, 0.040, 0.180},
+    {G3K_GEMM_QUAD128, 128, 128, 2, 0.54, {1.05, 1.21, 0}, 0.077, 0.168},
+    {G3K_GEMM_QUAD256, 256, 128, 2, 1.34, {1.74, 2.70, 0}, 0.035, 0.166},
+};
+
+double form_time(const FormTime &f, int N, int K, int n_mat, const int *M, int S, int cus) {
+    long long tiles = 0, sum = 0;
+    for (int m = 0; m < n_mat; m++) {
+        tiles += (M[m] + f.rows - 1) / f.rows;
+        sum += M[m];
+    }
+    const long long blocks = (N + f.tokens - 1) / f.tokens, wgs = tiles * blocks * S, slots = (long long)cus * f.per_cu;
+    // the quads walk stages of 32, the others chunks of 64
+    const int all = (K + 63) / 64;
+    const bool quad = f.kind == G3K_GEMM_QUAD128 || f.kind == G3K_GEMM_QUAD256;
+    const double chunks = quad ? K / 64.0 / S : (double)((all + S - 1) / S);
+    const long long full = wgs / slots, rest = wgs % slots;
+    double t = 2.27 + (double)full * (f.round + f.chunk[f.per_cu - 1] * chunks);
+    if (rest) t += f.round + f.chunk[(rest + cus - 1) / cus - 1] * chunks;
+    const double out_mb = 4e-6 * N * (double)sum;
+    t += f.w_read * 2e-6 * (double)sum * K * (double)blocks + f.out * out_mb;
+    return S > 1 ? t + 3.27 + 0.32 * S * out_mb : t;
+}
+
+}  // namespace
+
 // The kernel and its k splits for N tokens.
-// - Up to 128 tokens, or a product of up to 12 GFLOP issued, is a stream of W:
-//   GEGLU's many rows take 256-row workgroups, one per CU; the others 64-row
-//   ones, two per CU (one where a second launch has to add the splits and
-//   N <= 96: each split costs that launch its partial products).  Splits of
-//   less than two chunks gain nothing.
-// - Beyond, the 256 x 128 tiles: split z adds its part to the time of a round
-//   of n_cu workgroups (1.75 us per 64-wide chunk and 5 us around the K loop,
-//   measured with every CU busy) and its partial products (moved at about 8
-//   MB per us); the S with the least total is taken.
-// - GEGLU takes the tiles unsplit.
+// - GEGLU: up to 128 tokens the 256-row stream, split until there is a
+//   workgroup per CU; beyond, the tiles unsplit.
+// - Partial products that the consumer adds (the residual step, which reads
+//   them anyway): the 64-row stream up to 128 tokens or 12 GFLOP issued, split
+//   to two workgroups per CU; beyond, the tiles, whose split z adds its part to
+//   the time of a round of n_cu workgroups (1.75 us per 64-wide chunk and 5 us
+//   around the K loop, measured with every CU busy) and its partial products
+//   (moved at about 8 MB per us); the S with the least total is taken.
+// - Otherwise the form and S of the least time above.  The candidates: the
+//   64-row stream in the range just given, unless a second token block would
+//   read W from memory again (more than two workgroups of one block per CU);
+//   the 256-row stream for 49 to 128 tokens over many rows; the tiles, split
+//   beyond 128 tokens; the quads.  One rule for all of them left 710 of the
+//   5500 products 10 to 88% over the earlier 128 x 128 tiles (a batch's logits
+//   in one call, 128 tokens, 262208 x 2560: 772 us for 423; 1024 tokens,
+//   102400 x 96: 145 for 112); with the times 25 are, by at most 21%.
+//   A split has at least two chunks, and its partial products at most 256 MB.
 extern "C" void g3k_gemm_plan(int N, int K, int n_mat, const int *M, int geglu, int consumer_adds, int n_cu, int *kind,
                               int *ksplit) {
     long long sum = 0, tiles64 = 0, tiles256 = 0;
@@ -505,32 +662,66 @@ extern "C" void g3k_gemm_plan(int N, int K, int n_mat, const int *M, int geglu, 
     }
     const int chunks = (K + 63) / 64, most = chunks > 1 ? chunks / 2 : 1;
     const int cus = n_cu > 0 ? n_cu : 256;
-    long long S = 1;
-    if (N <= 128 || (!geglu && N <= 4096 && 4.0 * N * (double)sum * K <= 12e9)) {
-        if (geglu) {
-            *kind = G3K_GEMM_WIDE;
-            S = cus / tiles256;
-        } else {
-            *kind = G3K_GEMM_NARROW;
-            const int per = narrow_tokens(N);
-            S = (long long)cus * (!consumer_adds && N <= 96 ? 1 : 2) / (tiles64 * ((N + per - 1) / per));
-        }
-        if (S > most) S = most;
-        *ksplit = S < 1 ? 1 : (int)S;
+    const bool stream = N <= 128 || (N <= 4096 && 4.0 * N * (double)sum * K <= 12e9);
+    const long long tiles = tiles256 * ((N + BN - 1) / BN);
+    const int per = narrow_tokens(N);
+    const long long wgs64 = tiles64 * ((N + per - 1) / per);
+    auto bounded = [&](long long S) { return (int)(S < 1 ? 1 : S > most ? most : S); };
+    auto room = [&](int S) { return S == 1 || 4.0 * S * N * (double)sum <= 256e6; };
+    *kind = G3K_GEMM_TILE;
+    *ksplit = 1;
+    if (geglu) {
+        if (N > 128) return;
+        *kind = G3K_GEMM_WIDE;
+        *ksplit = bounded(cus / tiles256);
         return;
     }
-    *ksplit = 1;
-    *kind = G3K_GEMM_TILE;
-    if (geglu) return;
-    const long long tiles = tiles256 * ((N + BN - 1) / BN);
+    if (consumer_adds && stream) {
+        *kind = G3K_GEMM_NARROW;
+        *ksplit = bounded(2LL * cus / wgs64);
+        return;
+    }
     double best = 0.0;
-    for (int s = 1; s <= 16 && s <= most; s++) {
-        if (s > 1 && 4.0 * s * N * (double)sum > 256e6) break;   // bounded workspace
-        double t = (double)((tiles * s + cus - 1) / cus) * (1.75 * ((chunks + s - 1) / s) + 5.0);
-        if (s > 1) t += (double)s * N * (double)sum * 8.0 / 8e6 + (consumer_adds ? 0.0 : 3.0);
-        if (s == 1 || t < best) {
+    if (consumer_adds) {
+        for (int s = 1; s <= 16 && s <= most && room(s); s++) {
+            double t = (double)((tiles * s + cus - 1) / cus) * (1.75 * ((chunks + s - 1) / s) + 5.0);
+            if (s > 1) t += (double)s * N * (double)sum * 8.0 / 8e6;
+            if (s == 1 || t < best) {
+                best = t;
+                *ksplit = s;
+            }
+        }
+        return;
+    }
+    for (const FormTime &f : FORMS) {
+        int tried = 0;
+        auto consider = [&](int S) {
+            if (S == tried || !room(S)) return;
+            tried = S;
+            double t = form_time(f, N, K, n_mat, M, S, cus);
+            // whole 128-byte lines of W: the 64-row stream's fit is over its
+            // measured times there (5.2 M outputs at K = 512: 20 against 17)
+            if (f.kind == G3K_GEMM_NARROW && K % 64 == 0 && K >= 256) t *= 0.85;
+            if (best > 0.0 && t >= best) return;
             best = t;
-            *ksplit = s;
+            *kind = f.kind;
+            *ksplit = S;
+        };
+        switch (f.kind) {
+            case G3K_GEMM_NARROW:
+                if (!stream || f.tokens != per || (N > per && tiles64 > 2 * cus)) break;
+                for (int j = 0; j <= 3; j++) consider(bounded((long long)j * cus / wgs64));
+                break;
+            case G3K_GEMM_WIDE:
+                if (N <= 48 || N > f.tokens || N <= f.tokens - (f.tokens == 64 ? 16 : 32) || tiles256 <= cus / 4) break;
+                consider(1);
+                consider(bounded(cus / tiles256));
+                break;
+            case G3K_GEMM_TILE:
+                for (int s = 1; s <= 16 && s <= most && (s == 1 || N > 128); s++) consider(s);
+                break;
+            default:
+                consider(1);
         }
     }
 }
@@ -542,13 +733,13 @@ extern "C" int g3k_gemm(const g3k_gemm_args *a, void *stream) {
         return (int)hipErrorInvalidValue;
     if (a->n_mat < 1 || a->n_mat > G3K_MATVEC_MAX || (geglu && a->n_mat != 2) || (a->mode != 0 && !geglu))
         return (int)hipErrorInvalidValue;
-    if (a->kind < G3K_GEMM_TILE || a->kind > G3K_GEMM_NARROW) return (int)hipErrorInvalidValue;
+    if (a->kind < G3K_GEMM_TILE || a->kind > G3K_GEMM_QUAD256) return (int)hipErrorInvalidValue;
     // at least one 64-wide chunk per split; the grid's y and z limits
     const bool stream_w = a->kind == G3K_GEMM_WIDE || a->kind == G3K_GEMM_NARROW;
     if (S < 1 || S > (a->K + 63) / 64 || S > 65535 || a->N > (stream_w ? 16 : BN) * 65535)
         return (int)hipErrorInvalidValue;
     // GEGLU is applied to whole sums: through part, or by an unsplit tile kernel
-    if (geglu && (stream_w ? !a->part : (S != 1 || a->part))) return (int)hipErrorInvalidValue;
+    if (geglu && (stream_w ? !a->part : (S != 1 || a->part || a->kind != G3K_GEMM_TILE))) return (int)hipErrorInvalidValue;
     // 32-bit buffer offsets, including the rows of a last partial tile
     if ((size_t)(a->N + BN) * a->ldx * 2 >= (1ull << 32)) return (int)hipErrorInvalidValue;
     for (int m = 0; m < a->n_mat; m++) {

@@ -21,7 +21,7 @@ from helpers import DeviceBuffer, g3attn
 from test_attn_hostemu import Emu, built  # noqa: F401  (built: the emulator's build)
 
 G = g3attn()
-TILE, WIDE, NARROW = range(3)
+TILE, WIDE, NARROW, QUAD128, QUAD256 = range(5)
 
 
 def plan(N, K, M, geglu=0, consumer_adds=0, n_cu=256):
@@ -39,15 +39,34 @@ def test_plan_stays_in_the_launchers_limits(K):
         for M in ([4], [64], [2560], [262208], [2048, 1024, 1024], [256, 256, 256]):
             for adds in (0, 1):
                 kind, s = plan(N, K, M, 0, adds)
-                assert kind in (TILE, NARROW) and 1 <= s <= (K + 63) // 64, (N, M, kind, s)
-                if kind == NARROW:
-                    assert N <= 4096
+                assert 0 <= kind <= QUAD256 and 1 <= s <= (K + 63) // 64, (N, M, kind, s)
+                if kind in (NARROW, WIDE):
+                    assert N <= (4096 if kind == NARROW else 128)
+                if kind in (QUAD128, QUAD256):
+                    assert s == 1 and not adds
                 if s > 1:
                     assert 4 * s * N * sum(M) <= 256e6, (N, M, s)
         kind, s = plan(N, K, [10240, 10240], 1)
         assert 1 <= s <= (K + 63) // 64
         assert kind == (WIDE if N <= 128 else TILE)
         assert s == 1 or kind == WIDE
+
+
+@pytest.mark.parametrize("N,M,K,kinds", [
+    (128, 262208, 2560, (WIDE, TILE)), (100, 262208, 512, (WIDE, QUAD128, QUAD256)),   # W read once
+    (100, 30000, 2560, (WIDE,)), (100, 2560, 10240, (NARROW,)), (1, 262208, 2560, (NARROW,)),
+    (1024, 102400, 96, (QUAD256,)), (2048, 12368, 352, (QUAD256,)), (1024, 10240, 512, (QUAD128, QUAD256)),   # short rows
+    (2048, 10240, 2560, (TILE,)), (2048, 2560, 10240, (TILE,)),
+    (4097, 256, 512, (QUAD128, QUAD256))])
+def test_plan_takes_the_form_measured_fastest(N, M, K, kinds):
+    """Stand-alone products on either side of the rule's lines: the forms that
+    are within 5% of the fastest there."""
+    assert plan(N, K, [M])[0] in kinds, plan(N, K, [M])
+
+
+def test_plan_splits_where_the_sums_cost_less_than_they_save():
+    assert plan(1500, 2144, [5684])[1] == 1 and plan(64, 512, [256])[1] == 1
+    assert plan(384, 10240, [2560])[1] > 4 and plan(77, 10240, [2560])[1] > 1
 
 
 SHAPES = [(16, 64, 32), (17, 68, 96), (33, 60, 160), (65, 132, 64), (1, 4, 224), (97, 132, 352)]
@@ -62,11 +81,13 @@ def test_forms_on_the_emulated_machine(built, tmp_path, cus):  # noqa: F811
 
 
 def test_many_tokens_on_the_emulated_machine(built, tmp_path):  # noqa: F811
-    """Past the weight stream's token limit: the 256 x 128 tiles, with rows
-    and tokens that end inside one and a half chunk of K at the end."""
-    assert plan(4100, 96, [4])[0] == TILE
+    """Past the weight stream's token limit: tiles with rows and tokens that
+    end inside one, and half a chunk of K at the end."""
+    assert plan(4100, 96, [4])[0] not in (NARROW, WIDE)
     e = Emu(tmp_path)
     e.matmul(4100, 4, 96)
+    for kind in (TILE, QUAD128, QUAD256):
+        emu_gemm(e, kind, 1, 0, 132, 260, 96)
     e.run()
 
 
@@ -100,7 +121,7 @@ def emu_gemm(e, kind, ksplit, geglu, N, M, K):
 
 @pytest.mark.parametrize("fetch", ["early", "late"])
 @pytest.mark.parametrize("kind,geglu,N", [(WIDE, 1, n) for n in (32, 64, 96, 128)]
-                         + [(NARROW, 0, n) for n in (16, 32, 48, 64)] + [(TILE, 0, 128), (TILE, 1, 128)])
+                         + [(NARROW, 0, n) for n in (16, 32, 48, 64)] + [(TILE, 0, 128), (TILE, 1, 128), (QUAD128, 0, 128), (QUAD256, 0, 128)])
 def test_rings_turn_over(built, tmp_path, kind, geglu, N, fetch):  # noqa: F811
     """Each form with more chunks per split than its LDS rings have slots, so
     that every slot is refilled while others are read: 11 and 12 chunks (the
@@ -116,7 +137,8 @@ def test_rings_turn_over(built, tmp_path, kind, geglu, N, fetch):  # noqa: F811
 @pytest.mark.gpu
 @pytest.mark.parametrize("N,M,K", SHAPES + [
     (32, 4, 64), (64, 260, 2592), (77, 2560, 2592), (96, 132, 10240), (128, 2560, 2080), (129, 132, 96), (7, 8, 10240), (48, 2560, 10240),
-    (300, 2560, 10240), (1500, 1028, 2592), (4100, 4, 96), (4097, 260, 32)])
+    (300, 2560, 10240), (1500, 1028, 2592), (4100, 4, 96), (4097, 260, 32), (65, 16644, 544), (128, 30000, 1056),
+    (777, 16388, 96), (640, 12364, 352), (49, 30004, 2592), (80, 30004, 2592), (128, 30004, 2592)])
 def test_forms(N, M, K):
     rng = np.random.default_rng(N * 7 + M * 13 + K)
     W = ((rng.standard_normal((M, K)) / 64).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
