@@ -947,14 +947,20 @@ static int prefill_attention(g3attn_ctx *c, int layer, int start_pos, int n, con
     const long long ldk = ((long long)nk + 63) / 64 * 64;
     const size_t v_bytes = align256((size_t)Hkv * ldk * D * sizeof(uint16_t));
     const int pb = 16 * ((c->prefill_qpw == 32 ? 2 : 1)) * ((8 / (c->prefill_qpw == 32 ? 2 : 1)) / c->group);
-    const int S = c->prefill_ksplit ? c->prefill_ksplit
-                                    : prefill_splits(n, hist, nk, is_global ? INT_MAX / 2 : W, pb, Hkv, Hq, c->n_cu);
-    const size_t po_bytes = S > 1 ? align256((size_t)S * n * Hq * D * sizeof(float)) : 0;
-    const size_t pml_bytes = S > 1 ? align256((size_t)S * n * Hq * 2 * sizeof(float)) : 0;
+    int S = c->prefill_ksplit ? c->prefill_ksplit
+                              : prefill_splits(n, hist, nk, is_global ? INT_MAX / 2 : W, pb, Hkv, Hq, c->n_cu);
     /* the fp8 cross policy's key-scale bytes, one per staged key row */
     const size_t ks_bytes = x8 ? align256((size_t)Hkv * ldk) : 0;
     hipSetDevice(c->device);
-    int rc = grow_pf(c, 4 * v_bytes + ks_bytes + po_bytes + pml_bytes);
+    size_t po_bytes, pml_bytes;
+    int rc;
+    /* fewer splits where memory is too short for the parts of many */
+    for (;; S = 4) {
+        po_bytes = S > 1 ? align256((size_t)S * n * Hq * D * sizeof(float)) : 0;
+        pml_bytes = S > 1 ? align256((size_t)S * n * Hq * 2 * sizeof(float)) : 0;
+        rc = grow_pf(c, 4 * v_bytes + ks_bytes + po_bytes + pml_bytes);
+        if (rc != G3_ERR_OUT_OF_MEMORY || S <= 4) break;
+    }
     if (rc) return rc;
     unsigned char *ws = (unsigned char *)c->d_pf;
     uint16_t *kq = (uint16_t *)ws;
@@ -1447,9 +1453,21 @@ int g3attn_matmul_bf16_device(g3attn_ctx *c, float *C, const uint16_t *W, const 
     const size_t plane = align256((size_t)N * K * 2);
     int kind, ksplit;
     g3k_gemm_plan(N, K, 1, &M, 0, 0, c->n_cu, &kind, &ksplit);
-    const size_t part = ksplit > 1 ? (size_t)ksplit * N * M * sizeof(float) : 0;
+    size_t part = ksplit > 1 ? (size_t)ksplit * N * M * sizeof(float) : 0;
+    /* The split products only save time: where the buffer cannot grow for them
+     * (the stream is being captured, or memory is short) the product runs
+     * unsplit in the planes' room. */
+    if (part && 2 * plane + part > c->d_big_cap) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(c->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) part = 0;
+    }
     int rc = grow_buf(c, (float **)&c->d_big, &c->d_big_cap, 2 * plane + part, "matmul planes");
+    if (rc == G3_ERR_OUT_OF_MEMORY && part) {
+        part = 0;
+        rc = grow_buf(c, (float **)&c->d_big, &c->d_big_cap, 2 * plane, "matmul planes");
+    }
     if (rc) return rc;
+    if (!part) ksplit = 1;
     uint16_t *xh = (uint16_t *)c->d_big, *xl = (uint16_t *)((unsigned char *)c->d_big + plane);
     g3k_rows_args r;
     memset(&r, 0, sizeof r);

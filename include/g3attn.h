@@ -316,7 +316,11 @@ int g3attn_prefill_tokens(g3attn_ctx *ctx, const int *tokens, int num_tokens, in
  * X [N][K] fp32, W [M][K] bf16, C [N][M] fp32, device pointers; M a multiple
  * of 4, K of 32.  On MFMA: X is split into bf16 hi + lo planes (relative error
  * <= 2^-17) and both are multiplied by W with fp32 accumulation.  Enqueued on
- * the context stream. */
+ * the context stream.  The planes, and the partial products where K is split,
+ * live in a workspace that grows with N, K and M; where it cannot grow for the
+ * latter (out of memory, or under stream capture) the product runs unsplit.  A
+ * captured call holds the workspace's address: a later call that grows it
+ * makes the graph invalid. */
 int g3attn_matmul_bf16_device(g3attn_ctx *ctx, float *C, const uint16_t *W, const float *X, int N, int M, int K);
 
 /* gemma3_transformer_prefill_batched (gemma3_transformer.c:526-787) on the

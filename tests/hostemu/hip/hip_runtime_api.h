@@ -63,6 +63,8 @@ hipError_t hipMemset(void *p, int value, size_t bytes);
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned flags);
 hipError_t hipStreamDestroy(hipStream_t s);
 hipError_t hipStreamSynchronize(hipStream_t s);
+typedef enum hipStreamCaptureStatus { hipStreamCaptureStatusNone = 0 } hipStreamCaptureStatus;
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *status);
 
 hipError_t hipEventCreate(hipEvent_t *e);
 hipError_t hipEventDestroy(hipEvent_t e);

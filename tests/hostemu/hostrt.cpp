@@ -114,9 +114,11 @@ hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t attr, int device) 
 }
 hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
 
+// HOSTEMU_MALLOC_MAX: a larger allocation fails, as on a full device.
 hipError_t hipMalloc(void **p, size_t bytes) {
     g_alloc_calls++;
-    *p = aligned(bytes);
+    const char *most = std::getenv("HOSTEMU_MALLOC_MAX");
+    *p = most && bytes > std::strtoull(most, nullptr, 10) ? nullptr : aligned(bytes);
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipFree(void *p) {
@@ -160,6 +162,10 @@ hipError_t hipStreamDestroy(hipStream_t s) {
     return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *status) {
+    *status = hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
 
 hipError_t hipEventCreate(hipEvent_t *e) {
     *e = new hostemu_event{0.0, false};

@@ -91,6 +91,20 @@ def test_many_tokens_on_the_emulated_machine(built, tmp_path):  # noqa: F811
     e.run()
 
 
+def test_unsplit_where_memory_is_short(built, tmp_path):  # noqa: F811
+    """The split products only save time: 100 tokens into 64 rows of 2304, 18
+    splits of 25 KiB beside 900 KiB of planes, run unsplit on a device whose
+    largest allocation is 1 MB; with room a second launch adds them."""
+    assert plan(100, 2304, [64])[1] == 18
+    for room, reduces in ((1000000, 0), (1 << 40, 1)):
+        d = tmp_path / str(room)
+        d.mkdir()
+        e = Emu(d, H=1, Hkv=1, max_context=32)
+        e.matmul(100, 64, 2304)
+        launches = e.run(HOSTEMU_MALLOC_MAX=room)
+        assert launches.get("split_reduce_kernel", (0, 0))[0] == reduces, launches
+
+
 def emu_gemm(e, kind, ksplit, geglu, N, M, K):
     """One g3k_gemm of a given form on the emulated machine, against fp64."""
     W = [(e.rng.standard_normal((M, K)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16) for _ in range(1 + geglu)]
@@ -152,6 +166,53 @@ def test_forms(N, M, K):
     ratio = float(np.max(np.abs(got - X64 @ W64.T) / bound))
     print(f"[gemm forms] N={N} M={M} K={K} plan={plan(N, K, [M])} max err / bound = {ratio:.3f}", flush=True)
     assert np.all(np.isfinite(got)) and ratio <= 1.0
+
+
+@pytest.mark.gpu
+def test_captured_where_the_workspace_cannot_grow():
+    """A product recorded into a HIP graph after an eager call whose workspace
+    holds the planes but not this one's split products: it runs unsplit instead
+    of allocating under capture.  Three replays, new activations and an eager
+    call of the first product before each, against fp64."""
+    hip, vp = DeviceBuffer.hip(), C.c_void_p
+    hip.hipStreamBeginCapture.argtypes = [vp, C.c_int]
+    hip.hipStreamEndCapture.argtypes = [vp, C.POINTER(vp)]
+    hip.hipGraphInstantiate.argtypes = [C.POINTER(vp), vp, vp, vp, C.c_size_t]
+    hip.hipGraphLaunch.argtypes = [vp, vp]
+    for f in ("hipGraphExecDestroy", "hipGraphDestroy"):
+        getattr(hip, f).argtypes = [vp]
+    N, M, K, small = 40, 1024, 2592, 8
+    assert plan(N, K, [M])[1] * M > 4 * plan(N, K, [small])[1] * small   # its parts do not fit
+    rng = np.random.default_rng(40)
+    W = ((rng.standard_normal((M, K)) / 64).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    W64 = (W.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    with G.Context(G.default_config(max_context=256, num_layers=6), 256) as ctx:
+        dW, dX, dC, dS = DeviceBuffer.of(W), DeviceBuffer(N * K * 4), DeviceBuffer(N * M * 4), DeviceBuffer(N * small * 4)
+        stream, graph, exe = vp(ctx.stream()), vp(), vp()
+
+        def eager():
+            ctx.matmul_bf16_device(dS.ptr, dW.ptr, dX.ptr, N, small, K)
+            ctx.synchronize()
+
+        dX.upload(np.zeros((N, K), np.float32))
+        eager()
+        assert hip.hipStreamBeginCapture(stream, 2) == 0     # hipStreamCaptureModeRelaxed
+        ctx.matmul_bf16_device(dC.ptr, dW.ptr, dX.ptr, N, M, K)
+        assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, 0) == 0
+        for rep in range(3):
+            X = rng.standard_normal((N, K)).astype(np.float32)
+            dX.upload(X)
+            eager()
+            assert hip.hipGraphLaunch(exe, stream) == 0
+            ctx.synchronize()
+            X64 = X.astype(np.float64)
+            bound = (2.0 ** -16 + K * 2.0 ** -24) * (np.abs(X64) @ np.abs(W64).T)
+            for buf, m in ((dC, M), (dS, small)):
+                got = buf.download(np.float32, (N, m)).astype(np.float64)
+                assert np.all(np.abs(got - X64 @ W64[:m].T) <= bound[:, :m]), (rep, m)
+        hip.hipGraphExecDestroy(exe)
+        hip.hipGraphDestroy(graph)
 
 
 @pytest.mark.gpu

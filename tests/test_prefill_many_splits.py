@@ -29,6 +29,17 @@ def test_the_rules_empty_splits_fetch_nothing_out_of_range(built, tmp_path):  # 
     assert launches["prefill_kernel"] == (1, 16) and launches["prefill_merge_kernel"][0] == 1, launches
 
 
+def test_fewer_splits_where_memory_is_short(built, tmp_path):  # noqa: F811
+    """The same call on a device whose largest allocation holds the staged
+    keys and four splits' parts, but not sixteen's."""
+    e = Emu(tmp_path, H=1, Hkv=1, max_context=2056, window=64)
+    e.kv_append(5, 0, 2035)
+    e.prefill(5, 2035, 16)
+    staged = 2112 * 256 * 2 * 4
+    launches = e.run(HOSTEMU_MALLOC_MAX=staged + 8 * 16 * 256 * 4)
+    assert launches["prefill_kernel"] == (1, 4) and "prefill_merge_kernel" not in launches, launches
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("splits", [8, 16])
 def test_forced_split_counts(monkeypatch, splits):
