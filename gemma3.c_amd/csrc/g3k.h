@@ -217,7 +217,8 @@ typedef struct {
     float qscale;             /* softmax scale * log2(e) */
     int queries_per_wave;     /* 16 (8 waves, 2 per SIMD) or 32 (4 waves, 1 per SIMD) */
     int schedule;             /* 16 queries per wave: 0 = all waves in phase, 1 = SIMD pairs in opposite phase */
-    void *ev0, *ev1;          /* hipEvent_t: begin / end of prefill_kernel's dispatch, or NULL */
+    void *ev0, *ev1;          /* hipEvent_t: begin of prefill_kernel's dispatch and end of the one that writes the
+                               * output (its own, or the merge's), or NULL */
     /* Key splits (1, 2, 4, 8 or 16).  With S > 1 every (query block, KV head) runs as
      * S workgroups over consecutive parts of its key tiles; each writes its
      * unnormalised O and (max, sum) per query row to part_o [S][n][H_q][D]

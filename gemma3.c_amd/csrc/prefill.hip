@@ -974,17 +974,19 @@ hipError_t launch_prefill(const g3k_prefill_args *a, hipStream_t st) {
     constexpr int PB = 16 * NQB * ((8 / NQB) / G);
     const int nqb = (a->n + PB - 1) / PB;
     const dim3 grid(nqb * a->n_kv_heads * a->ksplit);
-    // With timing events the dispatch itself records them (kernel begin / end).
+    const bool merge = a->ksplit > PREFILL_MERGE_IN;
+    // With timing events the dispatches themselves record them: the kernel's
+    // begin, and the end of the one that writes the output.
+    const hipEvent_t ev0 = (hipEvent_t)a->ev0, ev1 = merge ? nullptr : (hipEvent_t)a->ev1;
     if (a->kscale)
-        hipExtLaunchKernelGGL((prefill_kernel<G, NQB, true>), grid, dim3(512 / NQB), 0, st, (hipEvent_t)a->ev0,
-                              (hipEvent_t)a->ev1, 0, *a);
+        hipExtLaunchKernelGGL((prefill_kernel<G, NQB, true>), grid, dim3(512 / NQB), 0, st, ev0, ev1, 0, *a);
     else
-        hipExtLaunchKernelGGL((prefill_kernel<G, NQB, false>), grid, dim3(512 / NQB), 0, st, (hipEvent_t)a->ev0,
-                              (hipEvent_t)a->ev1, 0, *a);
+        hipExtLaunchKernelGGL((prefill_kernel<G, NQB, false>), grid, dim3(512 / NQB), 0, st, ev0, ev1, 0, *a);
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess || a->ksplit <= PREFILL_MERGE_IN) return e;
+    if (e != hipSuccess || !merge) return e;
     const long long waves = (long long)a->n * a->n_kv_heads * a->group;
-    hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(NT), 0, st, *a);
+    hipExtLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(NT), 0, st, nullptr,
+                          (hipEvent_t)a->ev1, 0, *a);
     return hipGetLastError();
 }
 

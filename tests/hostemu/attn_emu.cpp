@@ -36,6 +36,8 @@
 //   forward_device token pos logits|-           (the device copies)
 //   forward_token token pos logits              (the uploaded model)
 //   prefill_tokens n tokens start logits        (the uploaded model)
+//   profile kind       (g3attn_profile_enable, or once enabled
+//                    g3attn_profile_read: prints "profile <kind> <ms> <count>")
 //   destroy
 //   front_stage_only Hkv nk V vt_out            (g3k_rope_write_stage with an
 //                    empty batch, ra.n = 0, and no cache: the V^T staging of
@@ -161,6 +163,7 @@ int main(int argc, char **argv) {
     std::ifstream script(g_dir + "/script.txt");
     if (!script) die("no script.txt");
     g3attn_ctx *ctx = nullptr;
+    bool profiling = false;
     int H = 0, Hkv = 0, layers = 0, hidden = 0, vocab = 0;
     Model *model = nullptr;
     const size_t D = 256;
@@ -444,6 +447,18 @@ int main(int argc, char **argv) {
             std::vector<float> logits((size_t)vocab, -12345.0f);
             check(g3attn_prefill_tokens(ctx, tokens.data(), n, start, logits.data()), cmd);
             write_bin(lf, logits.data(), logits.size());
+        } else if (cmd == "profile") {
+            int kind, count = 0;
+            double ms = 0.0;
+            in >> kind;
+            if (!in || !ctx) die("bad profile line");
+            if (!profiling) {
+                profiling = true;
+                check(g3attn_profile_enable(ctx, 1), cmd);
+            } else {
+                check(g3attn_profile_read(ctx, kind, &ms, &count), cmd);
+                std::printf("profile %d %.3f %d\n", kind, ms, count);
+            }
         } else if (cmd == "front_stage_only") {
             // The front launch with no batch tokens must stage V^T and touch
             // nothing of the (absent) cache destination.

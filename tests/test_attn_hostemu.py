@@ -253,6 +253,7 @@ class Emu:
         # "launch <kernel expression> <launches> <workgroups> <threads> <ms>":
         # (launches, workgroups summed over them), keyed by the bare kernel
         # name; self.threads[name]: threads per workgroup of the last launch
+        self.stdout = res.stdout
         launches = {}
         for ln in res.stdout.splitlines():
             if ln.startswith("launch "):

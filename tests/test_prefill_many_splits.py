@@ -40,6 +40,24 @@ def test_fewer_splits_where_memory_is_short(built, tmp_path):  # noqa: F811
     assert launches["prefill_kernel"] == (1, 4) and "prefill_merge_kernel" not in launches, launches
 
 
+@pytest.mark.parametrize("splits", [4, 8])
+def test_profiled_time_covers_the_merge(built, tmp_path, splits):  # noqa: F811
+    """g3attn_profile_read's kind 1 is the time to the finished output on
+    either side of four splits: the merge is inside the kernel up to four, and
+    its own launch beyond."""
+    e = Emu(tmp_path, H=1, Hkv=1, max_context=640, window=64)
+    e.lines.append("profile 1")
+    e.prefill(5, 0, 400)
+    e.lines.append("profile 1")
+    e.run(G3ATTN_PREFILL_SPLITS=splits)
+    ms = {ln.split()[1].strip("()").split("<")[0]: float(ln.split()[-1]) for ln in e.stdout.splitlines()
+          if ln.startswith("launch prefill_") or ln.startswith("launch (prefill_")}
+    profiled = [ln.split()[1:] for ln in e.stdout.splitlines() if ln.startswith("profile ")]
+    assert len(ms) == (2 if splits > 4 else 1), ms
+    assert profiled[0][0] == "1" and int(profiled[0][2]) == 1
+    assert float(profiled[0][1]) >= sum(ms.values()) - 0.2, (profiled, ms)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("splits", [8, 16])
 def test_forced_split_counts(monkeypatch, splits):
