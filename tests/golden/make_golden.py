@@ -7,6 +7,9 @@ present at build time; that library is the reference's own code compiled in
 place by oracle/Makefile (never copied).  Inputs come from the oracle's
 seeded generator; each fixture stores the FNV-1a hashes of its inputs so
 generator drift on another machine is caught before outputs are compared.
+The *_case / *_inputs functions, which the tests call on any machine, take the
+RoPE tables from the oracle's restatement, whose bits rope.npz pins to the
+reference's.
 
     python tests/golden/make_golden.py            # all fixtures
     python tests/golden/make_golden.py --no-big   # skip the configs[3] run (~1-2 min)
@@ -99,7 +102,7 @@ def decode_case(config, layer, pos, max_context):
     """Inputs of one decode step; the cache holds normed + RoPE'd keys of the
     earlier positions the layer keeps (reference cache layout)."""
     cfg = O.Config(max_context=max_context)
-    table = O.rope_table(max_context, cfg.theta(layer), use_ref=True)
+    table = O.rope_table(max_context, cfg.theta(layer))
     is_g = O.is_global_layer(layer)
     lo = 0 if is_g else max(0, pos - cfg.sliding_window)
     n = pos - lo
@@ -132,7 +135,7 @@ def decode_fixture():
 
 def prefill_inputs(config, start, n, layer, max_context=8192):
     cfg = O.Config(max_context=max_context)
-    table = O.rope_table(max_context, cfg.theta(layer), use_ref=True)
+    table = O.rope_table(max_context, cfg.theta(layer))
     s = lambda t: O.seed_for(config, t)
     Q = O.gen_normal_bf16(n * QS, s(1), start * QS).reshape(n, QS)
     K = O.gen_normal_bf16(n * KS, s(2), start * KS).reshape(n, KS)
@@ -203,7 +206,7 @@ def layer_attention_case(layer, pos, hidden=2560):
     wq, wk, wv = (weights_bf16(r, hidden, s) for r, s in ((2048, 0x9100), (1024, 0x9200), (1024, 0x9300)))
     wo = weights_bf16(hidden, 2048, 0x9400)
     x = O.gen_normal_bf16(hidden, 0x9500 + pos)
-    table = O.rope_table(8192, cfg.theta(layer), use_ref=True)
+    table = O.rope_table(8192, cfg.theta(layer))
     is_g = O.is_global_layer(layer)
     lo = 0 if is_g else max(0, pos - cfg.sliding_window)
     n = pos - lo
