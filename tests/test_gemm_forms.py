@@ -251,22 +251,26 @@ def test_gate_up_token_classes(n, hidden):
     batched_against_token_loop(n, hidden, 288)
 
 
-def batched_against_token_loop(n, hidden, inter):
-    vocab = 96
-    rng = np.random.default_rng(hidden)
-
+def random_model(rng, hidden, inter, vocab, layers):
+    """Host weights of a small model at the default 8 / 4 heads of 256."""
     def w(*shape, scale):
         return ((rng.standard_normal(shape) * scale).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
 
     s = 1 / np.sqrt(hidden)
-    layer = dict(input_layernorm=w(hidden, scale=0.1), q_proj=w(2048, hidden, scale=s), k_proj=w(1024, hidden, scale=s),
-                 v_proj=w(1024, hidden, scale=s), o_proj=w(hidden, 2048, scale=0.02), q_norm=w(256, scale=0.1),
-                 k_norm=w(256, scale=0.1), post_attention_layernorm=w(hidden, scale=0.1),
-                 gate_proj=w(inter, hidden, scale=s), up_proj=w(inter, hidden, scale=s),
-                 down_proj=w(hidden, inter, scale=0.1), pre_feedforward_layernorm=w(hidden, scale=0.1),
-                 post_feedforward_layernorm=w(hidden, scale=0.1))
+    layers = [dict(input_layernorm=w(hidden, scale=0.1), q_proj=w(2048, hidden, scale=s), k_proj=w(1024, hidden, scale=s),
+                   v_proj=w(1024, hidden, scale=s), o_proj=w(hidden, 2048, scale=0.02), q_norm=w(256, scale=0.1),
+                   k_norm=w(256, scale=0.1), post_attention_layernorm=w(hidden, scale=0.1),
+                   gate_proj=w(inter, hidden, scale=s), up_proj=w(inter, hidden, scale=s),
+                   down_proj=w(hidden, inter, scale=0.1), pre_feedforward_layernorm=w(hidden, scale=0.1),
+                   post_feedforward_layernorm=w(hidden, scale=0.1)) for _ in range(layers)]
+    return G.host_weights(w(vocab, hidden, scale=1.0), layers, w(hidden, scale=0.1))
+
+
+def batched_against_token_loop(n, hidden, inter):
+    vocab = 96
+    rng = np.random.default_rng(hidden)
+    HW, keep = random_model(rng, hidden, inter, vocab, 1)
     tokens = rng.integers(0, vocab, n).astype(np.int32)
-    HW, keep = G.host_weights(w(vocab, hidden, scale=1.0), [layer], w(hidden, scale=0.1))
     cfg = G.default_config(num_layers=1, hidden_size=hidden, intermediate_size=inter, vocab_size=vocab, max_context=max(64, n))
     with G.Context(cfg, max(64, n)) as ctx:
         ctx.upload_weights(HW)

@@ -1,12 +1,15 @@
 """Prefill with 8 and 16 key splits, merged by a second launch (few query
 blocks over many keys): forced counts that leave splits empty, and the counts
 the split rule takes for a short batch after a long history, each against the
-oracle at the path's 2e-3 x RMS bar, repeated bit for bit."""
+oracle at the path's 2e-3 x RMS bar, repeated bit for bit; and the same counts
+inside the whole model's batched prefill, where the merge writes o_proj's bf16
+planes, against the token forward."""
 import numpy as np
 import pytest
 
 from helpers import TOL, rel_err
-from test_attn_hostemu import Emu, built  # noqa: F401  (built: the emulator's build)
+from test_attn_hostemu import Emu, _emu_for, _forward_model, built  # noqa: F401  (built: the emulator's build)
+from test_gemm_forms import G, random_model
 
 
 @pytest.mark.parametrize("splits", [8, 16])
@@ -89,3 +92,48 @@ def test_the_rule_takes_them_after_a_long_history():
         want, _, _ = case.oracle()
         assert rel_err(got, want) <= TOL
         assert np.array_equal(got, case.gpu(c))
+
+
+@pytest.mark.parametrize("splits", [8, 16])
+def test_planes_on_the_emulated_machine(built, tmp_path, splits):  # noqa: F811
+    """Two chunks through the small model, the second after history, with the
+    merge writing the attention output as planes in every layer: the last
+    token's logits at the token forward's 1e-4 x RMS."""
+    f, embed, layers, norm, tokens, want = _forward_model(32)
+    e = _emu_for(tmp_path, f)
+    e.model(embed, layers, norm)
+    e.lines.append("upload")
+    e._save("a.bin", tokens[:16].astype(np.int32))
+    e._save("b.bin", tokens[16:].astype(np.int32))
+    e.logits("prefill_tokens", "16 a.bin 0", want[15], "first chunk")
+    e.logits("prefill_tokens", "16 b.bin 16", want[31], "second chunk")
+    launches = e.run(G3ATTN_PREFILL_SPLITS=splits)
+    assert launches["prefill_merge_kernel"][0] == 2 * f["layers"], launches
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("start,n,forced", [(947, 77, None), (4000, 64, None), (300, 40, 8), (300, 40, 16)])
+def test_planes_in_the_model(monkeypatch, start, n, forced):
+    """A follow-up chunk through six layers (five local, one global), at the
+    rule's own 8 or 16 splits and forced ones, against the token forward over
+    the same chunk on the same history.  Bar: the batched path's 1e-3 x RMS
+    (projections on two bf16 planes)."""
+    if forced:
+        monkeypatch.setenv("G3ATTN_PREFILL_SPLITS", str(forced))
+    rng = np.random.default_rng(start + n)
+    HW, keep = random_model(rng, 256, 512, 96, 6)
+    tokens = rng.integers(0, 96, start + n).astype(np.int32)
+    cfg = G.default_config(num_layers=6, hidden_size=256, intermediate_size=512, vocab_size=96, max_context=4096)
+    with G.Context(cfg, 4096) as ctx:
+        ctx.upload_weights(HW)
+        ctx.prefill_tokens(tokens[:start], logits=False)
+        got = ctx.prefill_tokens(tokens[start:], start_pos=start)
+        assert ctx.last_splits(1) in ((forced,) if forced else (8, 16)), ctx.last_splits(1)
+    with G.Context(cfg, 4096) as ctx:
+        ctx.upload_weights(HW)
+        ctx.prefill_tokens(tokens[:start], logits=False)
+        for i in range(start, start + n):
+            want = ctx.forward_token(tokens[i], i)
+    e = rel_err(got, want)
+    print(f"[planes start={start} n={n} forced={forced}] {e:.2e}", flush=True)
+    assert e <= 1e-3
