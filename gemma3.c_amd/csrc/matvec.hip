@@ -313,7 +313,9 @@ __global__ __launch_bounds__(NT) void matvec_kernel(g3k_matvec_args a) {
 // all) instead of one per 4 rows is what lets the gate / up launch carry the
 // residual step too: at hidden 2560 the step's own launch took 4.3 us, and
 // folded into 5120 one-shot workgroups it cost more than that.
-constexpr int FLOW_WGS = 512;
+#ifndef G3K_FLOW_WGS
+#define G3K_FLOW_WGS 512                     // resident workgroups (a small grid in a test build)
+#endif
 
 template <bool GEGLU, int NCH>
 __global__ __launch_bounds__(NT, 2) void matvec_flow_kernel(g3k_matvec_args a) {
@@ -407,7 +409,7 @@ hipError_t launch_flow_n(const g3k_matvec_args *a, hipStream_t st) {
     long long items = a->M[0];
     for (int m = 1; m < a->n_mat && !GEGLU; m++) items += a->M[m];
     const long long wgs = (items + NW - 1) / NW;
-    hipLaunchKernelGGL((matvec_flow_kernel<GEGLU, NCH>), dim3((unsigned)(wgs < FLOW_WGS ? wgs : FLOW_WGS)), dim3(NT), 0,
+    hipLaunchKernelGGL((matvec_flow_kernel<GEGLU, NCH>), dim3((unsigned)(wgs < G3K_FLOW_WGS ? wgs : G3K_FLOW_WGS)), dim3(NT), 0,
                        st, *a);
     return hipGetLastError();
 }

@@ -7,7 +7,10 @@ Every layout the launcher picks is driven: one row per wave (Q/K/V, K =
 GEGLU pair, and the scalar path (K not a multiple of 8, or x unaligned).  The
 residual prologue (g3k_matvec_args.pre_*: x = rmsnorm(r + rmsnorm(t, w_post),
 w_next), formed by every workgroup, the new residual stored by workgroup 0)
-runs with both gains, with the post-norm absent, and on the GEGLU launch.
+runs with both gains, with the post-norm absent, and on the GEGLU launch.  On
+the vector path the prologue's launch is the resident form, whose waves keep
+two or three items in registers: a build with one workgroup drives every
+length of its loop and tail.
 
 The expected values come from the oracle: gemma3_matvec_bf16
 (gemma3_kernels.c:188-238), gemma3_rmsnorm_bf16 (:289-304) and
@@ -45,7 +48,7 @@ def _bf16(rng, n, scale):
     return (x.view(np.uint32) >> 16).astype(np.uint16)
 
 
-def _run(tmp, mats, K, mode=0, x=None, pre=None, x_off=0, eps=1e-6):
+def _run(tmp, mats, K, mode=0, x=None, pre=None, x_off=0, eps=1e-6, exe=EXE):
     os.makedirs(tmp, exist_ok=True)
     for m, A in enumerate(mats):
         np.ascontiguousarray(A, np.uint16).tofile(os.path.join(tmp, f"A{m}.bin"))
@@ -66,7 +69,7 @@ def _run(tmp, mats, K, mode=0, x=None, pre=None, x_off=0, eps=1e-6):
         f.write(f"{mode} {len(mats)} {K} {M[0]} {M[1]} {M[2]} {int(pre is not None)} {has_wp} {has_wn} "
                 f"{x_off} {float(np.float32(eps))!r}\n")
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=1", UBSAN_OPTIONS="print_stacktrace=1")
-    res = subprocess.run([EXE, tmp], capture_output=True, text=True, timeout=600, env=env)
+    res = subprocess.run([exe, tmp], capture_output=True, text=True, timeout=600, env=env)
     assert res.returncode == 0 and "matvec_emu: ok" in res.stdout, res.stderr[-4000:]
     assert "runtime error" not in res.stderr and "AddressSanitizer" not in res.stderr, res.stderr[-4000:]
     n_out = 1 if mode == GEGLU else len(mats)
@@ -107,9 +110,10 @@ def test_unaligned_x_takes_the_scalar_path(built, tmp_path):
 
 @pytest.mark.parametrize("K,post", [(2560, True), (512, False)])
 def test_three_matrices_with_residual_prologue(built, tmp_path, K, post):
-    """The Q/K/V launch with the residual step in its prologue: three
-    matrices sharing x, x formed by every workgroup, the new residual stored
-    once.  K 512 without the post-norm takes the split-over-waves layout."""
+    """The Q/K/V launch with the residual step in its prologue (the resident
+    form, at 5 chunks per lane and at 1): three matrices sharing x, x formed by
+    every workgroup, the new residual stored once, with and without the
+    post-norm."""
     rng = np.random.default_rng(K)
     mats = [_bf16(rng, M * K, 0.05).reshape(M, K) for M in (64, 32, 36)]
     t = rng.standard_normal(K).astype(np.float32)
@@ -123,6 +127,46 @@ def test_three_matrices_with_residual_prologue(built, tmp_path, K, post):
         err = rel_err(y, O.matvec_bf16(A, x))
         print(f"[hostemu matvec prologue] K={K} post={post} M={A.shape[0]} rel_err={err:.3e}")
         assert err < BAR
+
+
+@pytest.mark.parametrize("geglu", [False, True])
+@pytest.mark.parametrize("K", [512, 520, 2560, 3584, 4096])
+def test_resident_items_per_wave(built, tmp_path, K, geglu):
+    """One workgroup, so wave w of 4 takes items w, w + 4, ..: from one item per
+    wave to two whole rounds of the pipeline and every remainder (it holds 3
+    items, 2 for GEGLU above 3072), the last item of some waves missing, items
+    passing from one matrix to the next inside a round.  K: 1, 2, 5, 7 and 8
+    chunks per lane, the last one partly past the row's end at 520."""
+    rng = np.random.default_rng(K + geglu)
+    t, r = (rng.standard_normal(K).astype(np.float32) for _ in range(2))
+    wp, wn = _bf16(rng, K, 0.2), _bf16(rng, K, 0.2)
+    s, x = _prologue_oracle(t, r, wp, wn)
+    full = _bf16(rng, 2 * 40 * K, 0.05).reshape(2, 40, K)
+    x64 = x.astype(np.float64)
+
+    def product(A):
+        """A x in fp64 and its fp32 bound: a lane adds up to 64 products, six
+        steps add the lanes, and x itself is a few roundings off (its two
+        norms): under 96 x 2^-24 of the sum of magnitudes."""
+        A64 = (A.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+        return A64 @ x64, 96 * 2.0 ** -24 * (np.abs(A64) @ np.abs(x64))
+
+    for items in (1, 4, 6, 8, 11, 12, 16, 19, 20, 24, 27, 28, 32, 35, 36, 38):
+        if geglu:
+            mats = [full[0, :items], full[1, :items]]
+            (g, bg), (u, bu) = product(mats[0]), product(mats[1])
+            gelu = 0.5 * g * (1 + np.tanh(0.7978845608028654 * (g + 0.044715 * g ** 3)))
+            # |gelu'| <= 1.13; gelu itself to 8 x 2^-24 of |g|
+            want = [(gelu * u, 1.13 * bg * (np.abs(u) + bu) + np.abs(gelu) * bu + 8 * 2.0 ** -24 * np.abs(g * u))]
+        else:
+            cut = [0, items] if items < 3 else [0, items // 2, items // 2 + 1, items]
+            mats = [full[0, a:b] for a, b in zip(cut, cut[1:])]
+            want = [product(A) for A in mats]
+        ys, r_out = _run(str(tmp_path / str(items)), mats, K, mode=GEGLU if geglu else 0, pre=(t, r, wp, wn),
+                         exe=EXE + "_flow1")
+        assert rel_err(r_out, s) < BAR
+        for y, (w, bound) in zip(ys, want):
+            assert np.all(np.abs(y - w) <= bound), (items, float(np.max(np.abs(y - w) / bound)))
 
 
 @pytest.mark.parametrize("K", [100, 12])
