@@ -247,8 +247,19 @@ def test_row_lengths(hidden):
 @pytest.mark.parametrize("n,hidden", [(16, 32), (64, 96), (65, 64), (96, 1056), (97, 2080), (128, 96)])
 def test_gate_up_token_classes(n, hidden):
     """Gate and up as a weight stream at the edges of its token classes (32,
-    64, 96 and 128 per workgroup), from one chunk of K to many."""
+    64, 96 and 128 per workgroup), one to three chunks of K per split."""
     batched_against_token_loop(n, hidden, 288)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [32, 64, 96, 128])
+def test_gate_up_rings_turn_over(n):
+    """The same classes at Gemma3-4B's sizes, where a split walks 13 or 14
+    chunks through rings of two and three slots: the counted waits in their
+    steady state, against the token forward."""
+    kind, splits = plan(n, 2560, [10240, 10240], 1)
+    assert kind == WIDE and 40 // splits >= 8
+    batched_against_token_loop(n, 2560, 10240)
 
 
 def random_model(rng, hidden, inter, vocab, layers):
