@@ -516,10 +516,10 @@ def test_token_forward(built, tmp_path, fold):
     norms, the fused Q/K/V GEMV with or without the residual prologue,
     decode, o_proj, GEGLU, down_proj, tied logits): each token's logits
     against the oracle's gemma3_transformer_forward
-    (gemma3_transformer.c:396-512), for each residual-fold mode.  Fold 1
-    (the default) runs 11 tokens, wrapping the 8-row window; the others 3.
+    (gemma3_transformer.c:396-512), for each residual-fold mode.  Folds 1 and
+    3 (the default) run 11 tokens, wrapping the 8-row window; 0 runs 3.
     Bar 1e-4 x RMS, as on the GPU."""
-    n = 11 if fold == 1 else 3
+    n = 11 if fold else 3
     f, embed, layers, norm, tokens, want = _forward_model(n)
     e = _emu_for(tmp_path, f)
     e.model(embed, layers, norm)

@@ -90,8 +90,8 @@ def test_forward_matches_reference_golden():
 def test_forward_fold_modes(fold, monkeypatch):
     """The residual step between two GEMVs (post-norm, residual add, next
     pre-norm) as the one-workgroup kernel (G3ATTN_FORWARD_FOLD=0), in the
-    prologue of the next layer's Q/K/V launch (1, the default), or also in
-    the gate/up launch's (3): every step's logits and the final hidden state
+    prologue of the next layer's Q/K/V launch (1), or also in the gate/up
+    launch's (3, the default): every step's logits and the final hidden state
     against the oracle.  Layer 2's input norm sits 2 bytes past an 8-byte
     boundary, so the fold into layer 2's Q/K/V launch falls back to the
     kernel for that step, and the residual stream still comes out right."""
