@@ -100,23 +100,19 @@ __device__ __forceinline__ float *out_base(const g3k_gemm_args &a, int m, int z,
 // Many tokens: 256 weight rows (GEGLU: 128 gate rows and the same 128 up
 // rows) x 128 tokens per workgroup of 8 waves, one workgroup per CU, K in
 // chunks of 64 with two chunks of LDS (2 x 64 KiB).  The eight waves are four
-// 128-row x 64-token quarters times two halves of every chunk's k values:
-// each wave reads 16 fragments for 64 MFMAs (as a 128 x 64 wave tile does
-// with 128 accumulator registers), two waves run per SIMD, and a fetch takes
-// whole 128-byte lines (8 rows x 128 B) instead of half lines (16 rows x 64
-// B, whose 64-byte requests halve what an L2 delivers).  The two k halves
-// meet through LDS at the end, each wave finishing half of its pair's tiles.
-// Split-K (ksplit) fills the chip where the tiles alone do not.
-// Against 128- and 256-row x 128-token tiles with 32-wide stages, two
-// workgroups per CU (us, Gemma3-4B shapes): 8192 tokens: Q/K/V 349 -> 338,
-// o_proj 185 -> 180, down_proj 896 -> 781; 2048: 88 -> 72, 56 -> 54, 300 ->
-// 193; 512: 53 -> 26, 22 -> 22, 79 -> 62; gate + up at 256 / 512 / 1024 / 2048
-// / 8192: 97 -> 72, 136 -> 128, 248 -> 205, 447 -> 382, 1509 -> 1422 (1.21
-// PFLOP/s issued, what a library bf16 product of that size reaches here).
-// A single 64-wide stage per workgroup and two of them per CU in turn measured
-// the same at 8192 and slower below (gate + up 407 at 2048).  The K loop is bound by the matrix cores at the clocks they
-// sustain and by the L2 -> LDS stream about equally (down_proj at 8192
-// without its fetches: 602 us; with a quarter of its MFMAs: 645).
+// 128-row x 64-token quarters times two halves of every chunk's k values: a
+// wave reads 16 fragments for 64 MFMAs, two waves run per SIMD, and a fetch
+// takes whole 128-byte lines (8 rows x 128 B; 16 rows x 64 B halve what an L2
+// delivers).  The two k halves meet through LDS at the end, each wave
+// finishing half of its pair's tiles.
+// Against Quads' tiles (us): down_proj (2560 x 10240) of 8192 / 2048 / 512
+// tokens 896 -> 781, 300 -> 193, 79 -> 62; gate and up (2 x 10240 x 2560) of
+// 8192 / 2048 / 256 tokens 1509 -> 1422 (1.21 PFLOP/s issued, what a library
+// bf16 product of that size reaches here), 447 -> 382, 97 -> 72.  One 64-wide
+// stage and two such workgroups per CU: the same at 8192, slower below (gate
+// and up of 2048: 407).  The K loop is bound by the matrix cores at the clocks
+// they sustain and by the L2 -> LDS stream about equally (down_proj at 8192
+// without its fetches: 602; with a quarter of its MFMAs: 645).
 template <bool GEGLU>
 struct Pairs {
     static constexpr int THREADS = 512, WAVES = 2;
@@ -226,7 +222,7 @@ __device__ __forceinline__ void Pairs<GEGLU>::run(const g3k_gemm_args &a) {
             for (int nt = 0; nt < NTL; nt++) {
                 const int n = n0 + wn * 64 + nt * 16 + fr;
                 f32x4 v = in[(t * NTL + nt) * 64];
-                v = hw ? v + acc[mt][nt] : acc[mt][nt] + v;
+                v += acc[mt][nt];
                 if (GEGLU) {
                     const f32x4 u = acc[tile(hw, t + 2)][nt] + in[((t + 2) * NTL + nt) * 64];
                     if (n < N && m < M)   // M is a multiple of 4 (checked on the host)

@@ -266,7 +266,7 @@ __device__ __forceinline__ int vswz(int d) { return (d >> 2) & 3; }
 // bank group of a chunk is its index % 16, and kswz maps each read set onto
 // all 16 values.  It replaced 1040-byte padded rows: the kernel's LDS
 // bank-conflict cycles fell from 4.0 to 1.33 per LDS instruction and
-// configs[3] from 588.6 to 578.6 us on one box.
+// 8192 tokens of a global layer from 588.6 to 578.6 us on one card.
 __device__ __forceinline__ int kswz(int r) { return ((r >> 3) << 2) | (r & 3); }
 
 // Raw buffer descriptor over [base, base + bytes): stride 0, the gfx9
@@ -359,8 +359,8 @@ __device__ __forceinline__ void tile_scores(f32x4 (&s)[NQB][2], const unsigned c
 #pragma unroll
     for (int t = 0; t < PF; t++) load(f[t], t);
     // issue priority for the score MFMAs over the other wave of the SIMD
-    // (its softmax and P.V): configs[3] 580.5 -> 570.8 us, configs[2]
-    // 52.7 -> 51.9 us; the same around the P.V MFMAs gained nothing
+    // (its softmax and P.V): 8192 tokens, global: 580.5 -> 570.8 us,
+    // 2048, local: 52.7 -> 51.9 us; the same around the P.V MFMAs gained nothing
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int t = 0; t < 8; t++) {
@@ -823,7 +823,7 @@ __device__ __forceinline__ void attend(const g3k_prefill_args &p, unsigned char 
         // which go to and come from the point of coherence shared by all
         // XCDs, so no cache-wide writeback or invalidate is needed.  (An
         // agent-scope __threadfence does both to the XCD's whole L2; with
-        // one per workgroup configs[2] took 188 us instead of 53.)  The
+        // one per workgroup 2048 local tokens took 188 us, not 53.)  The
         // parts of split s of this block are one run of PB * H_q rows: one
         // descriptor per split, offsets relative to the block's first token.
         auto part_rsrc = [&](int sp) {

@@ -606,7 +606,7 @@ int g3attn_upload_rope(g3attn_ctx *c, const float *rope_local, const float *rope
  * where H_kv is a multiple of 8, else one query head per workgroup (H_q a
  * multiple of 8; each KV head's rows are then read once per query head, by
  * workgroups on different XCDs).  On MI355X at 8 query / 4 KV heads the one
- * query head per workgroup took configs[0] from 8.6 to 7.2-7.4 us per call;
+ * query head per workgroup took 512 local rows from 8.6 to 7.2-7.4 us per call;
  * whole groups on 4 XCDs (the other 4 idle) took 9.9 us.  Global layers
  * (G3ATTN_DECODE_XMERGE=2 admits them) would read their long caches twice. */
 static int xm_heads(const g3attn_ctx *c, int n_splits, int is_global) {
@@ -672,7 +672,7 @@ static int decode_enqueue(g3attn_ctx *c, int layer, int pos, const float *q, con
      * from evicting everything else.  Called for attention alone, a local
      * layer re-reads a window that changes by one row per token, so its rows
      * are loaded normally and the memory-side cache keeps them (29 + 5 stack
-     * at 131071: 1089 -> 1079 us per token; configs[0] 9.4 -> 8.9 us).
+     * at 131071: 1089 -> 1079 us per token; 512 local rows 9.4 -> 8.9 us).
      * Inside the token forward the 28-29 windows (235 MB) would instead push
      * out the norm rows the residual steps re-read every token (local
      * decode -0.4 us, residual step +0.5 us: 2.10 -> 2.12 ms per token), so

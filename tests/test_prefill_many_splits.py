@@ -116,8 +116,7 @@ def test_planes_on_the_emulated_machine(built, tmp_path, splits):  # noqa: F811
 def test_planes_in_the_model(monkeypatch, start, n, forced):
     """A follow-up chunk through six layers (five local, one global), at the
     rule's own 8 or 16 splits and forced ones, against the token forward over
-    the same chunk on the same history.  Bar: the batched path's 1e-3 x RMS
-    (projections on two bf16 planes)."""
+    the same chunk on the same history, at 1e-4 x RMS (2e-6 measured)."""
     if forced:
         monkeypatch.setenv("G3ATTN_PREFILL_SPLITS", str(forced))
     rng = np.random.default_rng(start + n)
@@ -136,4 +135,4 @@ def test_planes_in_the_model(monkeypatch, start, n, forced):
             want = ctx.forward_token(tokens[i], i)
     e = rel_err(got, want)
     print(f"[planes start={start} n={n} forced={forced}] {e:.2e}", flush=True)
-    assert e <= 1e-3
+    assert e <= 1e-4
