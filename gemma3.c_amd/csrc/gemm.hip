@@ -635,7 +635,10 @@ double form_time(const FormTime &f, int N, int K, int n_mat, const int *M, int S
 //   workgroup per CU; beyond, the tiles unsplit.
 // - Partial products that the consumer adds (the residual step, which reads
 //   them anyway): the 64-row stream up to 128 tokens or 12 GFLOP issued, split
-//   to two workgroups per CU; beyond, the tiles, whose split z adds its part to
+//   to two workgroups per CU (it is ahead there, 384 tokens of 2560 x 2560 take
+//   20 us against 27, level with the tiles from 13 to 20 and behind from 27
+//   GFLOP: 256 tokens of 2560 x 10240 51 against 47, 1024 of 2560 x 2560 40
+//   against 39); beyond, the tiles, whose split z adds its part to
 //   the time of a round of n_cu workgroups (1.75 us per 64-wide chunk and 5 us
 //   around the K loop, measured with every CU busy) and its partial products
 //   (moved at about 8 MB per us); the S with the least total is taken.
